@@ -241,11 +241,13 @@ static size_t plan_bytes_estimate(const Plan& p)
         b += vox * 4 + (size_t)p.vol_y * p.max_subset * p.sino_stride * sb;
         b += n * p.vol_z * 8 + n * p.proj * 8 + (size_t)p.vol_x * p.vol_z * 4;
         b += n * (size_t)(p.vol_z * 2.5 + 16) * 16;  // FP sample tables (bounded by 60 deg)
+        // back-projection tiles: every tilt is in the initial list and in a subset's
+        b += 2 * n * (size_t)bp_ztiles(p.vol_z, 8) * BP_WAVES * ((p.vol_x + BP_TX - 1) / BP_TX) * sizeof(int2);
     } else {
         b += (size_t)p.wbp_slab * 3 * p.vol_z * (p.vol_x / 2 + 1) * sizeof(float2);
         b += (size_t)p.wbp_slab * 4 * p.vol_z * p.vol_x * sizeof(float);
         b += n * 2 * p.vol_z * 8 + n * 16;
-        b += n * (size_t)((2 * p.vol_z + BP_TZ - 1) / BP_TZ) * ((2 * p.vol_x + BP_TX - 1) / BP_TX) * 16;
+        b += n * (size_t)bp_ztiles(2 * p.vol_z, 8) * BP_WAVES * ((2 * p.vol_x + BP_TX - 1) / BP_TX) * sizeof(int2);
     }
     return b;
 }
@@ -273,7 +275,13 @@ static atr_status sart_tables_host(Plan& p, int tz, int chunk, int bz, int pf)
     p.bp_tz = tz;
     p.bp_chunk = chunk;
     p.fp_pf = fp_mode_supported(pf, p.vol_x) ? pf : 0;
-    build_bp_tiles(g.cos_sin, g.bp_lohi, p.n, p.vol_x, p.vol_z, 1.0, p.proj / 2.0, tz, g.bp_tiles);
+    std::vector<TiltRow> rows = p.all_tilts;
+    rows.insert(rows.end(), p.subset_tilts.begin(), p.subset_tilts.end());
+    const std::vector<BpTilt> lists = bp_list(g.cos_sin, rows, 1.0f);
+    std::vector<int> ends(1, (int)p.all_tilts.size());
+    for (int sb = 0; sb < p.n_subsets; sb++) ends.push_back(ends[0] + p.subset_off[sb + 1]);
+    build_bp_tiles(lists, ends, g.cos_sin, g.bp_lohi, p.vol_x, p.vol_z, 1.0, p.proj / 2.0, tz,
+                   g.bp_tiles);
     if (!build_fp_tables(g.cos_sin, p.n, p.vol_x, p.vol_z, p.proj, bz, g))
         return fail(ATR_ERR_INVALID_ARG, "SART needs every tilt in (-90, 90) degrees");
     std::vector<int>& sched = p.host.sched;
@@ -317,12 +325,11 @@ static atr_status sart_tables_device(Plan& p)
     std::vector<FpArgs>& fpa = p.host.fp_args;
     bpa.clear();
     fpa.clear();
-    bpa.push_back(bp_args(p, p.d_sino, p.n, p.d_lists, n_all, 1.0f, true));
+    bpa.push_back(bp_args(p, p.d_sino, p.n, 0, n_all, 1.0f, true));
     for (int s = 0; s < p.n_subsets; s++) {
         const int b0 = p.subset_off[s], b1 = p.subset_off[s + 1];
         const int f0 = p.subset_fp_off[s], f1 = p.subset_fp_off[s + 1];
-        bpa.push_back(bp_args(p, p.d_diff, p.max_subset, p.d_lists + n_all + b0, b1 - b0, p.relax,
-                              false));
+        bpa.push_back(bp_args(p, p.d_diff, p.max_subset, n_all + b0, b1 - b0, p.relax, false));
         fpa.push_back(fp_args(p, p.d_fp_lists + f0, f1 - f0, p.d_fp_pairs + p.subset_pair_off[s]));
     }
     if ((st = reupload(p, &p.d_bp_args, bpa, B, p.tab_bytes[7])) != ATR_OK) return st;
@@ -382,9 +389,15 @@ static atr_status plan_host(Plan& p)
     }
     if (p.method == ATR_METHOD_SART) {
         build_bp_intervals(g.cos_sin, p.n, p.vol_x, p.vol_z, p.proj, g.bp_lohi);
-        h.lists = p.all_tilts;
-        h.lists.insert(h.lists.end(), p.subset_tilts.begin(), p.subset_tilts.end());
+        std::vector<TiltRow> rows = p.all_tilts;
+        rows.insert(rows.end(), p.subset_tilts.begin(), p.subset_tilts.end());
+        h.lists = bp_list(g.cos_sin, rows, 1.0f);
+        h.lists.resize(h.lists.size() + BP_PAD);
         fill_table(d.fill_seed ^ 0x5A5A5A5A5A5A5A5Aull, p.vol_x * p.vol_z, h.fill_vol);
+        // back-projection tiles: a stage as large as a subset of up to 8 tilts
+        // (2-5 % less than 16 tilts a stage at 5 to 6 tilts, 3 % more at 12)
+        p.bp_tz = bp_default_tz(p.vol_x, p.vol_y, p.vol_z);
+        p.bp_chunk = p.max_subset <= 8 ? 8 : 16;
         // default forward-projector staging: register prefetch where it is
         // built (VolX 1024, 2048: measured faster at the full band height),
         // else direct
@@ -395,8 +408,11 @@ static atr_status plan_host(Plan& p)
     build_wbp_intervals(g.cos_sin, p.n, p.vol_x, p.vol_z, p.proj, g.wbp_lohi);
     // 2x-grid back-projection: tile windows/classes (excluded tilts are left
     // out of the list, GBackProjWbp.cu:31)
-    build_bp_tiles(g.cos_sin, g.wbp_lohi, p.n, 2 * p.vol_x, 2 * p.vol_z, 0.5,
-                   (double)(p.proj / 2) + 0.5, BP_TZ, h.wbp_tiles);
+    p.bp_tz = bp_default_tz(2 * p.vol_x, std::min(p.wbp_slab, p.vol_y), 2 * p.vol_z);
+    h.lists = bp_list(g.cos_sin, p.all_tilts, 0.5f);
+    build_bp_tiles(h.lists, {(int)p.all_tilts.size()}, g.cos_sin, g.wbp_lohi, 2 * p.vol_x,
+                   2 * p.vol_z, 0.5, (double)(p.proj / 2) + 0.5, p.bp_tz, h.wbp_tiles);
+    h.lists.resize(h.lists.size() + BP_PAD);
     h.filter = ramp_filter(p.proj);
     make_fft(p.proj, p.fft_proj);
     make_fft(2 * p.vol_x, p.fft_x2);
@@ -461,7 +477,7 @@ static atr_status plan_device(Plan& p)
     } else {
         if ((st = upload(p, &p.d_wbp_lohi, g.wbp_lohi, B)) != ATR_OK) return st;
         if ((st = upload(p, &p.d_wbp_tiles, h.wbp_tiles, B)) != ATR_OK) return st;
-        if ((st = upload(p, &p.d_lists, p.all_tilts, B)) != ATR_OK) return st;
+        if ((st = upload(p, &p.d_lists, h.lists, B)) != ATR_OK) return st;
         if ((st = dalloc(p, (void**)&p.d_wbp_grid,
                          (size_t)p.wbp_slab * 4 * p.vol_z * p.vol_x * sizeof(float), B)) != ATR_OK)
             return st;
@@ -475,15 +491,13 @@ static atr_status plan_device(Plan& p)
             a.proj = p.proj;
             a.list = p.d_lists;
             a.n_list = (int)p.all_tilts.size();
-            a.cs = p.d_cs;
             a.lohi = p.d_wbp_lohi;
+            a.lohi_stride = bp_zpad(2 * p.vol_z);
             a.tiles = p.d_wbp_tiles;
-            a.n_ztiles = (2 * p.vol_z + BP_TZ - 1) / BP_TZ;
+            a.n_ztiles = bp_ztiles(2 * p.vol_z, p.bp_tz);
             a.n_xtiles = (2 * p.vol_x + BP_TX - 1) / BP_TX;
             a.relax = 1.0f;
             a.positivity = 0;
-            a.scale = 0.5f;
-            a.offset = (float)(p.proj / 2) + 0.5f;
             a.sflag = p.d_sflag + y0;
             a.vol = p.d_wbp_grid;
             a.vol_x = 2 * p.vol_x;
@@ -801,7 +815,7 @@ static atr_status plan_autotune(Plan& p, hipStream_t s, int* tz_out, int* chunk_
         }
         if (!bp_ok || !fp_ok) {
             // nothing launched: restore the default shape and report it
-            (void)sart_tables(p, BP_TZ, BP_CHUNK, bzs[0], 0);
+            (void)sart_tables(p, 16, 16, bzs[0], 0);
             return fail(ATR_ERR_HIP, "autotune: no candidate tile shape launched");
         }
         std::lock_guard<std::mutex> lk(g_tune_mu);

@@ -19,13 +19,32 @@ constexpr float kEmpty = -1e10f;
 constexpr float kSentinel = -1e30f;
 
 // ---- tile shapes ---------------------------------------------------------
-// SART back-projection: a workgroup owns BP_TX x BP_TZ voxels of one slice;
-// lane = x, each thread walks BP_TZ rows of z.
-constexpr int BP_TX = 256;
-constexpr int BP_TZ = 16;
-constexpr int BP_CHUNK = 16;                 // tilts staged in LDS at once
-constexpr int BP_WIN = BP_TX + BP_TZ + 16;   // staged pairs per tilt
-constexpr int bp_win(int tz) { return BP_TX + tz + 16; }
+// Back-projection: a workgroup of BP_WAVES waves owns BP_TX x (BP_WAVES tz)
+// voxels of one slice; lane = x, each thread walks tz rows of z.
+constexpr int BP_TX = 64;
+constexpr int BP_WAVES = 4;
+constexpr int BP_THREADS = 64 * BP_WAVES;
+constexpr int BP_WBP_CHUNK = 32;             // tilts staged in LDS at once, WBP grid
+constexpr int XCDS = 8;                      // workgroups go to the XCDs in turn
+// Slices from which one XCD takes all tiles of a slice (6 % of the
+// reconstruction at 475 and 1024 slices, even at 256 and 300, 3 % slower at 64
+// and 96, where the XCDs' shares are uneven).
+constexpr int BP_XCD_SLICES = 256;
+// Staged pairs per tilt, at least one for each lane: the tile spans at most
+// sqrt(63^2 + (4 tz - 1)^2) samples (half that on the WBP's 2x grid);
+// build_bp_tiles leaves 3 before its smallest coordinate, and 2 follow the
+// largest.
+constexpr int bp_win(int tz, bool wbp) { return wbp ? 64 : tz == 16 ? 96 : 80; }
+// rows per tilt of an interval table: whole tiles of either height
+inline int bp_zpad(int vol_z) { return (vol_z + 63) / 64 * 64; }
+inline int bp_ztiles(int vol_z, int tz) { return (vol_z + BP_WAVES * tz - 1) / (BP_WAVES * tz); }
+// Rows per thread unless tuned: 16, or 8 where 16 would leave fewer than four
+// workgroups per CU (few slices).
+inline int bp_default_tz(int vol_x, int vol_y, int vol_z)
+{
+    const long tiles = (long)((vol_x + BP_TX - 1) / BP_TX) * bp_ztiles(vol_z, 16) * vol_y;
+    return tiles < 1024 ? 8 : 16;
+}
 // Forward projection: a workgroup of FP_THREADS owns one slice and a group of
 // tilts; wave w takes the (tilt, 64-ray tile) pairs w, w+16, ... (FP_MAXP at
 // most), so every wave sees every tilt; the slice is streamed through LDS in
@@ -77,15 +96,24 @@ struct TiltRow {
     int tilt;
     int row;
 };
+// The same on the device, with the tilt's cos and sin (scaled to the grid's
+// coordinate).  Lists are padded by BP_PAD entries, and so are the tile
+// tables: the kernels read a chunk's entries past the end of a list.
+struct BpTilt {
+    float c, s;
+    int row, tilt;
+};
+constexpr int BP_PAD = 32;
 
 // FP64 geometry evaluated once per plan on the host.
 struct Geometry {
     std::vector<float> cos_sin;        // [2N] float, as CTomoBase.cpp:55-65
-    std::vector<int2> bp_lohi;         // [N][VolZ] x-interval of GBackProj inclusion
-    // [N][ztiles][xtiles] {window start, class 0 empty / 1 full / 2 partial,
-    // FP32 bits of u - start at the tile's first voxel, 0}
-    std::vector<int4> bp_tiles;
-    std::vector<int2> wbp_lohi;        // [N][2VolZ] x2-interval of GBackProjWbp inclusion
+    std::vector<int2> bp_lohi;         // [N][bp_zpad(VolZ)] x-interval of GBackProj inclusion
+    // per list of n tilts: [4 ztiles][xtiles][n], one entry per wave of a
+    // tile: {4 window start + class (0 empty / 1 full / 2 partial), FP32 bits
+    // of u - start - 1/2 at the wave's first voxel}
+    std::vector<int2> bp_tiles;
+    std::vector<int2> wbp_lohi;        // [N][bp_zpad(2VolZ)] x2-interval of GBackProjWbp inclusion
     std::vector<int2> fp_range;        // [N][P] first valid sample and count of each ray
     std::vector<int> fp_len;           // [N] ray length L
     std::vector<int> fp_geo_off;       // [N] offset into fp_geo
@@ -116,8 +144,8 @@ struct HostTables {
     std::vector<float> shifts, local, filter;
     std::vector<int> fill_aln, fill_vol, sched;
     std::vector<float2> tw_bin[4], tw_proj, tw_x2, tw_z2, tw_z, tw_x;
-    std::vector<TiltRow> lists;
-    std::vector<int4> wbp_tiles;
+    std::vector<BpTilt> lists;
+    std::vector<int2> wbp_tiles;
     std::vector<BpArgs> bp_args;   // kernel arguments of every step
     std::vector<FpArgs> fp_args;
 };
@@ -159,7 +187,7 @@ struct Plan {
     // device tables
     float2* d_cs = nullptr;
     int2* d_bp_lohi = nullptr;
-    int4* d_bp_tiles = nullptr;
+    int2* d_bp_tiles = nullptr;
     int2* d_wbp_lohi = nullptr;
     int2* d_fp_range = nullptr;
     int* d_fp_geo_off = nullptr;
@@ -167,7 +195,7 @@ struct Plan {
     float4* d_fp_geo = nullptr;
     int4* d_fp_desc = nullptr;
     int* d_fp_pairs = nullptr;        // per subset: FP wave schedules (fp_pair_schedule)
-    TiltRow* d_lists = nullptr;       // all_tilts then every subset's BP list
+    BpTilt* d_lists = nullptr;        // all_tilts then every subset's BP list
     int* d_fp_lists = nullptr;        // every subset's FP list
     int* d_fill_aln = nullptr;        // [aln_x*aln_y]
     int* d_fill_vol = nullptr;        // [vol_x*vol_z]
@@ -196,7 +224,7 @@ struct Plan {
     int* d_sflag = nullptr;           // [vol_y] sinogram slice holds sentinels
     int* d_vflag = nullptr;           // [vol_y] volume slice holds sentinels
     double* d_vstats = nullptr;       // [vol_y][2] fill statistics of volume slices
-    int bp_tz = BP_TZ, bp_chunk = BP_CHUNK;   // back-projection tile shape (autotuned)
+    int bp_tz = 16, bp_chunk = 16;    // back-projection tile shape (bp_default_tz, autotuned)
     int fp_pf = 0;                    // forward projector: 0 direct staging, FP_PF_DMA, FP_PF_REG (autotuned)
     // batches holding this plan: their item arrays and captured graphs point
     // at its tables, so the tables must not be rebuilt while this is > 0
@@ -205,7 +233,7 @@ struct Plan {
     BpArgs* d_bp_args = nullptr;      // SART step arguments: initial BP, then per subset
     FpArgs* d_fp_args = nullptr;      // per subset
     float* d_wbp_grid = nullptr;      // [slab][2VolZ][2VolX] the 2x-grid back-projection
-    int4* d_wbp_tiles = nullptr;      // [N][2VolZ/16][2VolX/256] as bp_tiles
+    int2* d_wbp_tiles = nullptr;      // the 2x grid's, as bp_tiles
     float2* d_wbp_t = nullptr;        // [slab][2VolZ][VolX/2+1]
     float2* d_wbp_u = nullptr;        // [slab][VolZ][VolX/2+1]
     int wbp_slab = 0;
@@ -226,15 +254,14 @@ struct Plan {
 struct BpArgs {
     const void* sino;          // [VolY][rows_per_slice][stride] storage type
     int rows_per_slice, stride, proj;
-    const TiltRow* list;
+    const BpTilt* list;
     int n_list;
-    const float2* cs;
-    const int2* lohi;          // [N][VolZ]
-    const int4* tiles;         // [N][ztiles][xtiles] {window start, class, u0 bits, 0}
+    int lohi_stride;
+    const int2* lohi;          // [N][lohi_stride]
+    const int2* tiles;         // [4 ztiles][xtiles][n_list], Geometry::bp_tiles
     int n_ztiles, n_xtiles;
     float relax;
     int positivity;
-    float scale, offset;       // u = scale (fx cos + fz sin) + offset (offset enters via the tile table)
     const int* sflag;          // NULL: the sinogram holds no empty samples
     float* vol;
     int vol_x, vol_z;
@@ -393,8 +420,11 @@ atr_status hip_fail(hipError_t e, const char* what);
 void cos_sin_table(const float* tilts, int n, std::vector<float>& cs);
 void build_bp_intervals(const std::vector<float>& cs, int n, int vol_x, int vol_z, int proj,
                         std::vector<int2>& lohi);
-void build_bp_tiles(const std::vector<float>& cs, const std::vector<int2>& lohi, int n, int vol_x,
-                    int vol_z, double scale, double offset, int tz, std::vector<int4>& tiles);
+std::vector<BpTilt> bp_list(const std::vector<float>& cs, const std::vector<TiltRow>& rows, float scale);
+// lists: tilts of every list one after another, ends: where each list ends
+void build_bp_tiles(const std::vector<BpTilt>& lists, const std::vector<int>& ends,
+                    const std::vector<float>& cs, const std::vector<int2>& lohi, int vol_x,
+                    int vol_z, double scale, double offset, int tz, std::vector<int2>& tiles);
 void build_wbp_intervals(const std::vector<float>& cs, int n, int vol_x, int vol_z, int proj,
                          std::vector<int2>& lohi);
 bool build_fp_tables(const std::vector<float>& cs, int n, int vol_x, int vol_z, int proj,
@@ -427,8 +457,9 @@ void launch_filter_wbp(const Plan& p, const float* in, hipStream_t s);
 void launch_zero(float* ptr, size_t n, hipStream_t s);
 void launch_zero_int(int* ptr, int n, hipStream_t s);
 int wbp_col_block(int vol_z);
-BpArgs bp_args(const Plan& p, const void* sino, int rows, const TiltRow* list, int n_list,
-               float relax, bool check_sent);
+// first: offset of the list in p.d_lists
+BpArgs bp_args(const Plan& p, const void* sino, int rows, int first, int n_list, float relax,
+               bool check_sent);
 FpArgs fp_args(const Plan& p, const int* fp_list, int n_list, const int* sched);
 size_t fp_lds_bytes(int bz, int vol_x, int pf = 0);
 // step 0: initial back-projection, 1 + s: subset s (arguments in p.d_bp_args)

@@ -84,7 +84,7 @@ static atr_status batch_build(atr_batch* b)
             const int n_all = (int)p.all_tilts.size();
             if (n_all == 0) continue;
             BpItem e{};
-            e.a = bp_args(p, p.d_sino, p.n, p.d_lists, n_all, 1.0f, true);
+            e.a = bp_args(p, p.d_sino, p.n, 0, n_all, 1.0f, true);
             e.n_items_y = bp_items_per_slice(e.a);
             e.shape = bp_shape(p.bp_tz, p.bp_chunk);
             ent.push_back({e, p.vol_y * e.n_items_y, (double)n_all * p.bp_tz});
@@ -108,7 +108,7 @@ static atr_status batch_build(atr_batch* b)
                                 (double)p.vol_x * p.vol_z * std::min(f.a.group, f1 - f0)});
                 if (b1 > b0) {
                     BpItem e{};
-                    e.a = bp_args(p, p.d_diff, p.max_subset, p.d_lists + n_all + b0, b1 - b0,
+                    e.a = bp_args(p, p.d_diff, p.max_subset, n_all + b0, b1 - b0,
                                   p.relax, false);
                     e.n_items_y = bp_items_per_slice(e.a);
                     e.shape = bp_shape(p.bp_tz, p.bp_chunk);

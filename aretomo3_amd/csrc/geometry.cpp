@@ -113,14 +113,15 @@ void parallel_for(int n, const std::function<void(int)>& fn) { parallel_tilts(n,
 void build_bp_intervals(const std::vector<float>& cs, int n, int vol_x, int vol_z, int proj,
                         std::vector<int2>& lohi)
 {
-    lohi.assign((size_t)n * vol_z, make_int2(vol_x, -1));
+    const int stride = bp_zpad(vol_z);
+    lohi.assign((size_t)n * stride, make_int2(vol_x, -1));
     const double cx = proj / 2.0;
     const int end_x = proj - 2;
     parallel_tilts(n, [&](int t) {
         double c = cs[2 * t], s = cs[2 * t + 1];
         for (int z = 0; z < vol_z; z++) {
             double fz = z - vol_z * 0.5;
-            lohi[(size_t)t * vol_z + z] = run_of(vol_x, [&](int x) {
+            lohi[(size_t)t * stride + z] = run_of(vol_x, [&](int x) {
                 double fx = x - vol_x * 0.5;
                 double u = fx * c + fz * s + cx;
                 return !(u < 0 || u > end_x);
@@ -129,42 +130,76 @@ void build_bp_intervals(const std::vector<float>& cs, int n, int vol_x, int vol_
     });
 }
 
-// Per (tilt, z-tile, x-tile) of a back-projection grid: the start w0 of the
-// window of BP_TX + tz + 16 row samples the tile stages, and the tile class
-// (1 = every voxel of the tile uses the tilt, 0 = none does, 2 = some do).
-// The grid coordinate is u = scale (fx cos + fz sin) + offset (SART: scale 1,
-// offset P/2; the WBP 2x grid: scale 1/2, offset P/2 + 1/2).
+// Back-projection tiles of BP_TX x (BP_WAVES tz) voxels: per wave (tz rows),
+// x-tile and tilt, the start w0 of the row window that the tile stages (the
+// same for its waves), the class of the wave's voxels (1 = every one uses the
+// tilt, 0 = none does, 2 = some do; 0 below the volume) and the coordinate of
+// its first one.  The grid coordinate is u = scale (fx cos + fz sin) + offset
+// (SART: scale 1, offset P/2; the WBP 2x grid: scale 1/2, offset P/2 + 1/2).
 // w0 = floor(min u over the tile corners) - 3 in FP64; the kernel's FP32
-// coordinates relative to w0 then stay in [2, window - 2] (the tile spans at
-// most scale ((BP_TX-1)|cos| + (tz-1)|sin|) in u).  The third field holds
-// the FP32 bits of u - w0 at the tile's first voxel (x0, z0), formed in FP64:
-// the kernel adds (x - x0) scale cos and k scale sin to it in FP32.
-void build_bp_tiles(const std::vector<float>& cs, const std::vector<int2>& lohi, int n, int vol_x,
-                    int vol_z, double scale, double offset, int tz, std::vector<int4>& tiles)
+// coordinates relative to w0 then stay in [2, window - 2].  The second field
+// holds the FP32 bits of u - w0 - 1/2 at the wave's first voxel, formed in
+// FP64: the kernel adds (x - x0) scale cos and k scale sin to it in FP32, and
+// rounding the sum to the nearest integer gives the cell.
+void build_bp_tiles(const std::vector<BpTilt>& lists, const std::vector<int>& ends,
+                    const std::vector<float>& cs, const std::vector<int2>& lohi, int vol_x,
+                    int vol_z, double scale, double offset, int tz, std::vector<int2>& tiles)
 {
-    int nzt = (vol_z + tz - 1) / tz, nxt = (vol_x + BP_TX - 1) / BP_TX;
-    tiles.assign((size_t)n * nzt * nxt, int4{0, 0, 0, 0});
-    for (int t = 0; t < n; t++) {
+    const int nzt = bp_ztiles(vol_z, tz), nxt = (vol_x + BP_TX - 1) / BP_TX;
+    const size_t per = (size_t)nzt * BP_WAVES * nxt;
+    const int total = ends.back(), stride = bp_zpad(vol_z);
+    tiles.assign(per * total + BP_PAD, int2{0, 0});
+    parallel_tilts(total, [&](int l) {
+        int first = 0, seg = 0;
+        while (ends[seg] <= l) first = ends[seg++];
+        const int len = ends[seg] - first, t = lists[l].tilt;
+        int2* out = tiles.data() + per * first + (l - first);
         const double c = cs[2 * t], s = cs[2 * t + 1];
-        for (int zt = 0; zt < nzt; zt++)
-            for (int xt = 0; xt < nxt; xt++) {
-                int x0 = xt * BP_TX, x1 = std::min(x0 + BP_TX, vol_x) - 1;
-                bool full = true, any = false;
-                for (int z = zt * tz; z < std::min((zt + 1) * tz, vol_z); z++) {
-                    int2 r = lohi[(size_t)t * vol_z + z];
-                    if (!(r.x <= x0 && r.y >= x1)) full = false;
-                    if (!(r.x > x1 || r.y < x0)) any = true;
+        const int2* lh = lohi.data() + (size_t)t * stride;
+        for (int zt = 0; zt < nzt; zt++) {
+            // per wave: the intervals' overlap and union over its rows
+            int in_lo[BP_WAVES], in_hi[BP_WAVES], any_lo[BP_WAVES], any_hi[BP_WAVES];
+            for (int w = 0; w < BP_WAVES; w++) {
+                const int z0 = (zt * BP_WAVES + w) * tz, z1 = std::min(z0 + tz, vol_z);
+                in_lo[w] = 0, in_hi[w] = z0 < vol_z ? vol_x : -1;
+                any_lo[w] = vol_x, any_hi[w] = -1;
+                for (int z = z0; z < z1; z++) {
+                    in_lo[w] = std::max(in_lo[w], lh[z].x);
+                    in_hi[w] = std::min(in_hi[w], lh[z].y);
+                    if (lh[z].y >= lh[z].x) {
+                        any_lo[w] = std::min(any_lo[w], lh[z].x);
+                        any_hi[w] = std::max(any_hi[w], lh[z].y);
+                    }
                 }
-                const double fx0 = x0 - vol_x * 0.5, fx1 = x1 - vol_x * 0.5;
-                const double fz0 = zt * tz - vol_z * 0.5, fz1 = fz0 + (tz - 1);
-                const double umin =
-                    offset + scale * (std::min(c * fx0, c * fx1) + std::min(s * fz0, s * fz1));
-                const int w0 = (int)std::floor(umin) - 3;
-                const float u00 = (float)(scale * (c * fx0 + s * fz0) + offset - w0);
-                tiles[((size_t)t * nzt + zt) * nxt + xt] =
-                    int4{w0, full ? 1 : (any ? 2 : 0), __builtin_bit_cast(int, u00), 0};
             }
-    }
+            const int zt0 = zt * BP_WAVES * tz;
+            const double fz0 = zt0 - vol_z * 0.5, fz1 = fz0 + (BP_WAVES * tz - 1);
+            const double sz = std::min(s * fz0, s * fz1);
+            for (int xt = 0; xt < nxt; xt++) {
+                const int x0 = xt * BP_TX, x1 = std::min(x0 + BP_TX, vol_x) - 1;
+                const double fx0 = x0 - vol_x * 0.5, fx1 = x1 - vol_x * 0.5;
+                const int w0 = (int)std::floor(offset + scale * (std::min(c * fx0, c * fx1) + sz)) - 3;
+                for (int w = 0; w < BP_WAVES; w++) {
+                    const int z0 = zt0 + w * tz;
+                    // (a tile between the rows' intervals counts as partial)
+                    const bool full = in_lo[w] <= x0 && in_hi[w] >= x1;
+                    const bool any = any_lo[w] <= x1 && any_hi[w] >= x0;
+                    const float u00 =
+                        (float)(scale * (c * fx0 + s * (z0 - vol_z * 0.5)) + offset - w0 - 0.5);
+                    out[((size_t)(zt * BP_WAVES + w) * nxt + xt) * len] =
+                        int2{4 * w0 + (full ? 1 : (any ? 2 : 0)), __builtin_bit_cast(int, u00)};
+                }
+            }
+        }
+    });
+}
+
+std::vector<BpTilt> bp_list(const std::vector<float>& cs, const std::vector<TiltRow>& rows, float scale)
+{
+    std::vector<BpTilt> v;
+    for (const TiltRow& r : rows)   // scale is 1 or 1/2: both products are exact
+        v.push_back(BpTilt{scale * cs[2 * r.tilt], scale * cs[2 * r.tilt + 1], r.row, r.tilt});
+    return v;
 }
 
 // Recon/GBackProjWbp.cu:23-36 on the 2x grid (vol_x2 = 2 VolX, vol_z2 =
@@ -173,14 +208,15 @@ void build_wbp_intervals(const std::vector<float>& cs, int n, int vol_x, int vol
                          std::vector<int2>& lohi)
 {
     const int vx2 = 2 * vol_x, vz2 = 2 * vol_z;
-    lohi.assign((size_t)n * vz2, make_int2(vx2, -1));
+    const int stride = bp_zpad(vz2);
+    lohi.assign((size_t)n * stride, make_int2(vx2, -1));
     const int cx = proj / 2;
     const int end_x = proj - 2;
     parallel_tilts(n, [&](int t) {
         double c = cs[2 * t], s = cs[2 * t + 1];
         for (int z = 0; z < vz2; z++) {
             double fz = z - vz2 / 2.0;
-            lohi[(size_t)t * vz2 + z] = run_of(vx2, [&](int x) {
+            lohi[(size_t)t * stride + z] = run_of(vx2, [&](int x) {
                 double fx = x - vx2 / 2.0;
                 double u = (fx * c + fz * s) / 2 + cx + 0.5;
                 return !(u < 0 || u > end_x);

@@ -444,7 +444,11 @@ template <typename S, bool SENT, int ROWB, bool PF = false, int RP = 0>
 __global__ __launch_bounds__(FP_THREADS) void k_for_proj_diff(const FpArgs* __restrict__ a)
 {
     extern __shared__ float2 band[];
-    fp_block<S, SENT, ROWB, PF, RP>(as_cptr(a), band, blockIdx.x, blockIdx.y);
+    // slices from the last to the first, the back-projections run from the
+    // first to the last: each launch begins with the slices that the one
+    // before it left in the 256 MB memory-side cache (1024^2 x 256: 1.140 ->
+    // 1.115 ms here, 0.569 -> 0.550 ms in the back-projection)
+    fp_block<S, SENT, ROWB, PF, RP>(as_cptr(a), band, blockIdx.x, gridDim.y - 1 - blockIdx.y);
 }
 
 // Forward projection + difference of many series in persistent launches:

@@ -193,238 +193,370 @@ __global__ __launch_bounds__(256) void k_weight(const float* __restrict__ in, si
 // ------------------------------------------------------------------------
 // SART back-projection (Recon/GBackProj.cu:12-60).
 //
-// Workgroup = BP_TX x TZ voxels of one slice, lane = x, each thread walks
-// TZ z-rows (TZ = 16 by default, 8 a tuning choice).  For each chunk of CH
-// tilts (16 or 8) the needed part of every
-// sinogram row is staged in LDS as pairs (p[i] - i d[i], d[i]), d[i] =
-// p[i+1]-p[i], so that one ds_read_b64 and one FMA with the window
-// coordinate itself give the linear interpolation (slices with empty samples
-// stage (p[i], d[i]) and weight d by the fraction).  Inclusion comes
-// from the FP64 interval tables: tiles the host classified as fully inside
-// skip all per-lane tests and count per tile; partial tiles test x against
-// the (tilt, z) interval.  Sums and counts are FP32/int per voxel, in tilt
-// order, as the reference.  Everything per tilt (list entry, cos/sin, the
-// tile's window start and class) is wave-uniform and read with scalar loads.
-// ------------------------------------------------------------------------
-// One tile: voxels x0 .. x0+BP_TX-1, z0 .. z0+TZ-1 of slice y.  Ends
-// after a barrier, with the LDS free for the next tile.
+// Workgroup = BP_TX x (BP_WAVES TZ) voxels of one slice (64 x 64 at TZ = 16),
+// lane = x, wave = a quarter of the rows, each thread walks TZ z-rows.  For
+// each chunk of CH tilts the part of every sinogram row that the tile can
+// reach (at most |cos| 63 + |sin| 63 samples and guards: 96 at TZ = 16) is
+// staged in LDS as pairs (A_i, d_i), d_i = q_{i+1} - q_i, A_i = q_i -
+// (i - 1/2) d_i, so that a voxel's value is the one FMA A_i + v d_i at
+// v = u - 1/2, u its coordinate in the window.  A square tile reaches the
+// fewest samples for its voxels: 0.023 pairs are staged per update, against
+// 0.070 for 256 x 16 voxels.
 //
-// SENT: the slice's sinogram rows may hold empty samples.  Without them the
-// staged pair of window index i is (q_i, d_i) with q_i = q(w0 + i) - i d_i,
-// so the interpolation at window coordinate u is the single FMA
-// q_i + u d_i (no fraction); with them the pair is (q(w0 + i), d_i) and the
-// value q + fract(u) d, whose sentinel test must see the exact -1e30 scale.
-template <typename S, int TZ, int CH, bool WBP, bool SENT>
-__device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, float2 (&pairs)[CH][bp_win(TZ)],
-                                             int xt, int zt, int y)
+// The cell index costs two instructions: v + (2^23 + window base) rounds v to
+// the nearest integer, which is floor(u), into the low bits of the float
+// (a tie, u an integer, may take the cell below: both give the same value),
+// and a 16-bit shift makes those bits the byte address.  Both, like FMAs and
+// adds on vector registers, are instructions of which the SIMD issues two at
+// a time, from two waves; conversions, 32-bit left shifts and anything with a
+// scalar operand issue one at a time (measured: 2.3 and 4 cycles per wave
+// instruction at four waves per SIMD).  All operands of an update are
+// therefore vector registers, and its five instructions take 11.5 cycles,
+// against 14.5 with a scalar slope, a conversion and a shift-add.
+//
+// Inclusion comes from the FP64 interval tables: tiles the host classified as
+// fully inside skip all per-lane tests and count per tile; partial tiles test
+// x against the (tilt, z) interval.  Sums and counts are FP32/int per voxel,
+// in tilt order, as the reference.  What a wave needs per tilt (coordinate of
+// its first voxel, cos, sin, class) is put into LDS with the rows and read
+// one tilt ahead, so no scalar-load latency stands between two tilts.
+//
+// 1024^2 x 256, 12 to 13 tilts: 0.55 ms a launch (0.895 with 256 x 16 voxel
+// tiles, scalar operands and a conversion per update); 4.0 TB/s of the 4.9 a
+// large copy reaches.  WBP grid of 512^2 x 128, 41 tilts: 0.71 ms (1.29).  What
+// bounds it is the LDS (one 8-byte read per update: 9 cycles per SIMD) beside
+// the 11.5 issue cycles of an update; 5 (WBP: 6) waves per SIMD hide the
+// staging loads and the barrier.
+// ------------------------------------------------------------------------
+template <int TZ, int CH, bool WBP>
+struct BpLds {
+    float2 pairs[CH * bp_win(TZ, WBP)];
+    // per wave and tilt: u - w0 - 1/2 at the wave's first voxel, scaled cos
+    // and sin, class; one spare entry, read ahead of the last tilt
+    float4 ent[BP_WAVES][CH + 1];
+};
+
+// Byte address of the pair that v (plus the 2^23 of cm) falls into.
+__device__ __forceinline__ unsigned bp_addr(float v, float cm)
 {
-    const gptr<const S> sino = (gptr<const S>)A->sino;
+    unsigned a;
+    asm("v_lshlrev_b16 %0, 3, %1" : "=v"(a) : "v"(v + cm));
+    return a;
+}
+
+// v0 + k ss with k as the instruction's literal (a constant in a scalar
+// register would halve the issue rate).
+template <int K>
+__device__ __forceinline__ float bp_coord(float ss, float v0)
+{
+    if constexpr (K == 0) return v0;
+    if constexpr (K == 1) return v0 + ss;
+    float r;
+    asm("v_fmamk_f32 %0, %1, %2, %3"
+        : "=v"(r)
+        : "v"(ss), "i"(__builtin_bit_cast(int, (float)K)), "v"(v0));
+    return r;
+}
+
+// Rows K0 .. K0 + 7 of a tilt that every voxel uses: the eight LDS reads go
+// out before the first value is needed.
+template <int K0, int TZ>
+__device__ __forceinline__ void bp_full8(const char* pairs, float ss, float v0, float cm,
+                                         float (&acc)[TZ])
+{
+    float v[8];
+    float2 pr[8];
+    v[0] = bp_coord<K0>(ss, v0);
+    v[1] = bp_coord<K0 + 1>(ss, v0);
+    v[2] = bp_coord<K0 + 2>(ss, v0);
+    v[3] = bp_coord<K0 + 3>(ss, v0);
+    v[4] = bp_coord<K0 + 4>(ss, v0);
+    v[5] = bp_coord<K0 + 5>(ss, v0);
+    v[6] = bp_coord<K0 + 6>(ss, v0);
+    v[7] = bp_coord<K0 + 7>(ss, v0);
+#pragma unroll
+    for (int k = 0; k < 8; k++) pr[k] = *(const float2*)(pairs + bp_addr(v[k], cm));
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc[K0 + k] += fmaf(v[k], pr[k].y, pr[k].x);
+}
+
+// The x-intervals of eight rows of one tilt, one scalar load.
+struct BpRows8 {
+    int2 r[8];
+};
+
+// One tile.  The caller puts a barrier between two tiles of a workgroup.
+//
+// SENT: the slice's sinogram rows may hold empty samples.  The staged pair is
+// then (q_i, d_i) and the value q + fract(u) d, whose sentinel test must see
+// the exact -1e30 scale.
+template <typename S, int TZ, int CH, bool WBP, bool SENT>
+__device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>& lds, int xt,
+                                             int zt, int y)
+{
+    constexpr int WIN = bp_win(TZ, WBP);
     const int rows_per_slice = A->rows_per_slice, stride = A->stride, proj = A->proj;
-    const cptr<TiltRow> list = as_cptr(A->list);
-    const int n_list = A->n_list;
-    const cptr<float2> cs = as_cptr(A->cs);
-    const cptr<int2> lohi = as_cptr(A->lohi);
-    const cptr<int4> tiles = as_cptr(A->tiles);
-    const int n_ztiles = A->n_ztiles, n_xtiles = A->n_xtiles;
+    const int n_list = A->n_list, n_xtiles = A->n_xtiles;
+    const int vol_x = A->vol_x, vol_z = A->vol_z;
     const float relax = A->relax;
     const int positivity = A->positivity;
-    const float scale = A->scale;
-    const gptr<float> vol = as_gptr(A->vol);
-    const int vol_x = A->vol_x, vol_z = A->vol_z;
-    int* vflag = A->vflag;
-    const int tid = threadIdx.x;
-    constexpr int WIN = bp_win(TZ);
-    const int x0 = xt * BP_TX, z0 = zt * TZ;
-    const int x = x0 + tid;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x0 = xt * BP_TX, zq = zt * BP_WAVES + wave, z0 = zq * TZ;
+    const bool live = z0 < vol_z;
+    const int x = x0 + lane;
     const int xc = min(x, vol_x - 1);
-    const gptr<float> vslice = vol + (size_t)y * vol_z * vol_x;
-    // the slice (and below, the slice's sinogram rows) as buffers: a voxel's
-    // row offset is a scalar, its column the lane's fixed byte offset
+    // the slice and its sinogram rows as buffers: a row offset is a scalar, a
+    // column the lane's fixed byte offset
+    const gptr<float> vslice = as_gptr(A->vol) + (size_t)y * vol_z * vol_x;
     const __amdgpu_buffer_rsrc_t vres =
         buffer_of((const void*)vslice, (size_t)vol_z * vol_x * sizeof(float));
     const int row_bytes = vol_x * (int)sizeof(float);
-
-    // the voxels this thread updates, loaded now and consumed at the end
-    // (the WBP grid is written, not updated)
-    float vold[TZ];
-#pragma unroll
-    for (int k = 0; k < TZ; k++)
-        vold[k] = WBP ? 0.0f
-                      : ldb<float>(vres, xc * (int)sizeof(float), min(z0 + k, vol_z - 1) * row_bytes);
-
-    float acc[TZ];
-    int cnt[TZ];
-#pragma unroll
-    for (int k = 0; k < TZ; k++) {
-        acc[k] = 0.0f;
-        cnt[k] = 0;
-    }
-    int full_cnt = 0;
-    const float xf = (float)(xc - x0);   // offset from the tile's first voxel
-    const gptr<const S> base = sino + (size_t)y * rows_per_slice * stride;
+    const gptr<const S> base = (gptr<const S>)A->sino + (size_t)y * rows_per_slice * stride;
     const __amdgpu_buffer_rsrc_t sres =
         buffer_of((const void*)base, (size_t)rows_per_slice * stride * sizeof(S));
-    const cptr<int4> tile_tab = tiles + (size_t)zt * n_xtiles + xt;
-    const size_t tilt_step = (size_t)n_ztiles * n_xtiles;
+    // window starts are those of the workgroup's tile (the same in the
+    // entries of all its waves); coordinates and classes are the wave's
+    const gptr<const int2> etab = as_gptr(A->tiles) + ((size_t)zq * n_xtiles + xt) * n_list;
+
+    float vold[TZ];
+    float acc[TZ];
+    // counts of the partial tiles, two 16-bit counts to a register
+    unsigned cnt[TZ / 2];
+#pragma unroll
+    for (int k = 0; k < TZ; k++) acc[k] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < TZ / 2; k++) cnt[k] = 0;
+    int full_cnt = 0;
+    bool partial = false;
+    const float xf = (float)(xc - x0);   // offset from the tile's first voxel
 
     for (int c0 = 0; c0 < n_list; c0 += CH) {
         const int nc = min(CH, n_list - c0);
-        // ---- stage the row segments.  Pair i of tilt j is (q(g), q(g+1) - q(g))
-        // at g = w0 + i, where q is the row extended linearly beyond its ends:
-        // q(g) = p[ga] + (g - ga) (p[ga+1] - p[ga]), ga = clamp(g, 0, P-2).
-        // Inside [0, P-2] that is the plain pair; at g = -1 it extrapolates, so
-        // a coordinate that FP32 rounding puts just below 0 still interpolates
-        // the first sample.  Pairs further out are only read by voxels the
-        // exact intervals exclude.  Four tilts' loads are issued before any
-        // pair is formed. ----
-        for (int h = 0; h < nc; h += 4) {
-            float pv[4][2], rv[4][2];
-            int gv[4][2];
+        if (c0 > 0) __syncthreads();
+        // ---- stage: wave w takes the ROUNDS tilts from w ROUNDS on.  Pair i
+        // of a row is (q(g), q(g+1) - q(g)) at g = w0 + i, where q is the row
+        // extended linearly beyond its ends: q(g) = p[ga] + (g - ga)
+        // (p[ga+1] - p[ga]), ga = clamp(g, 0, P-2).  Inside [0, P-2] that is
+        // the plain pair; at g = -1 it extrapolates, so a coordinate that FP32
+        // rounding puts just below 0 still interpolates the first sample.
+        // Pairs further out are only read by voxels the exact intervals
+        // exclude.  The first 64 pairs of a tilt take one wave instruction,
+        // the U others share one with those of GU - 1 more tilts.  Past the
+        // list's end the tables go on (into the next list, or their padding):
+        // what is staged for those slots is not read.  All loads are issued
+        // before a pair is formed, on every path alike. ----
+        constexpr int ROUNDS = CH / BP_WAVES;
+        constexpr int U = WIN > 64 ? WIN - 64 : 0, GU = U > 0 ? 64 / U : 1;
+        constexpr int UP = U > 0 ? (ROUNDS + GU - 1) / GU : 0, NP = ROUNDS + UP;
+        struct WindowStarts {
+            int2 e[ROUNDS];
+        };
+        struct Tilts {
+            BpTilt t[ROUNDS];
+        };
+        const int jw = wave * ROUNDS;
+        const WindowStarts ws =
+            ldc((cptr<WindowStarts>)(as_cptr(A->tiles) + ((size_t)zq * n_xtiles + xt) * n_list + c0 + jw));
+        const Tilts tl = ldc((cptr<Tilts>)(as_cptr(A->list) + c0 + jw));
+        float2 pv[NP];
+        int ga[NP], w0v[NP], slot[NP];
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const TiltRow tr = ldc(list + c0 + min(h + q, nc - 1));
-                const int w0 = tile_tab[(size_t)tr.tilt * tilt_step].x;
-                const int row_off = tr.row * stride * (int)sizeof(S);
-#pragma unroll
-                for (int m = 0; m < 2; m++) {
-                    const int g = w0 + tid + m * BP_TX;
-                    const int ga = min(max(g, 0), proj - 2);
-                    if (m == 0 || tid < WIN - BP_TX) {
-                        pv[q][m] = ldb<S>(sres, ga * (int)sizeof(S), row_off);
-                        rv[q][m] = ldb<S>(sres, (ga + 1) * (int)sizeof(S), row_off);
-                    }
-                    gv[q][m] = g - ga;
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                if (h + q >= nc) break;
-#pragma unroll
-                for (int m = 0; m < 2; m++) {
-                    if (m == 1 && tid >= WIN - BP_TX) break;
-                    float p = pv[q][m], r = rv[q][m];
-                    if constexpr (SENT && !std::is_same<S, float>::value) {
-                        // narrow storage cannot hold -1e30: widen its empty
-                        // marks (a slice without them has nothing to widen)
-                        const float thr = empty_threshold<S>();
-                        if (p <= thr) p = kSentinel;
-                        if (r <= thr) r = kSentinel;
-                    }
-                    const float d = r - p;
-                    // SENT: the extended value; else that minus i d
-                    const int gi = SENT ? gv[q][m] : gv[q][m] - (tid + m * BP_TX);
-                    pairs[h + q][tid + m * BP_TX] = make_float2(fmaf((float)gi, d, p), d);
-                }
-            }
-        }
-        __syncthreads();
-        // ---- accumulate ----
-        for (int j = 0; j < nc; j++) {
-            const TiltRow tr = ldc(list + c0 + j);
-            // {w0, class, u - w0 at the tile's first voxel}
-            const int4 tw = ldc(tile_tab + (size_t)tr.tilt * tilt_step);
-            const float2 sc = ldc(cs + tr.tilt);
-            // both loads issued together, before the class test
-            asm volatile("" ::"s"(tw.z), "s"(sc.x), "s"(sc.y));
-            if (tw.y == 0) continue;
-            // scale is 1 or 1/2: both products are exact
-            const float cc = scale * sc.x, ss = scale * sc.y;
-            const float u0 = fmaf(xf, cc, __int_as_float(tw.z));
-            const float2* pj = pairs[j];
-            if (tw.y == 1 && !SENT) {
-                full_cnt += 1;
-#pragma unroll
-                for (int k = 0; k < TZ; k++) {
-                    float u = fmaf((float)k, ss, u0);
-                    int i = (int)u;
-                    float2 pr = pj[i];
-                    acc[k] += fmaf(u, pr.y, pr.x);
-                }
-            } else if (!SENT) {
-                const cptr<int2> lh = lohi + (size_t)tr.tilt * vol_z;
-#pragma unroll
-                for (int k = 0; k < TZ; k++) {
-                    const int2 r = ldc(lh + min(z0 + k, vol_z - 1));
-                    float u = fmaf((float)k, ss, u0);
-                    int i = (int)u;
-                    float2 pr = pj[i];
-                    float v = fmaf(u, pr.y, pr.x);
-                    bool in = (x >= r.x) & (x <= r.y);
-                    acc[k] += in ? v : 0.0f;
-                    cnt[k] += in ? 1 : 0;
-                }
+        for (int q = 0; q < NP; q++) {
+            int w0, voff, soff = 0;
+            if (q < ROUNDS) {
+                w0 = ws.e[q].x >> 2;
+                slot[q] = (jw + q) * WIN + lane;
+                ga[q] = min(max(w0 + lane, 0), proj - 2);
+                voff = ga[q] * (int)sizeof(S);
+                soff = tl.t[q].row * stride * (int)sizeof(S);
             } else {
-                const cptr<int2> lh = lohi + (size_t)tr.tilt * vol_z;
+                // lanes U s .. U s + U - 1: the upper pairs of tilt
+                // (q - ROUNDS) GU + s (the last one again past the wave's)
+                const int s = lane / (U > 0 ? U : 64), i = 64 + lane % (U > 0 ? U : 64);
+                int row = 0, r = 0;
+                w0 = 0;
 #pragma unroll
-                for (int k = 0; k < TZ; k++) {
-                    const int2 r = ldc(lh + min(z0 + k, vol_z - 1));
-                    float u = fmaf((float)k, ss, u0);
-                    int i = (int)u;
-                    float f = __builtin_amdgcn_fractf(u);
-                    float2 pr = pj[i];
-                    float v = fmaf(f, pr.y, pr.x);
-                    bool in = (x >= r.x) & (x <= r.y) & !(v <= kEmpty);
-                    acc[k] += in ? v : 0.0f;
-                    cnt[k] += in ? 1 : 0;
+                for (int h = 0; h < GU; h++) {
+                    const int qq = min((q - ROUNDS) * GU + h, ROUNDS - 1);
+                    if (h == 0 || s >= h) {
+                        w0 = ws.e[qq].x >> 2;
+                        row = tl.t[qq].row;
+                        r = qq;
+                    }
+                }
+                slot[q] = (jw + r) * WIN + i;
+                ga[q] = min(max(w0 + i, 0), proj - 2);
+                voff = (row * stride + ga[q]) * (int)sizeof(S);
+            }
+            w0v[q] = w0;
+            pv[q] = ldb2<S>(sres, voff, soff);
+        }
+        if (lane < nc) {
+            const int2 e = ldgo(etab + c0 + lane);
+            const BpTilt bt = ldgo(as_gptr(A->list) + c0 + lane);
+            lds.ent[wave][lane] = make_float4(__int_as_float(e.y), bt.c, bt.s,
+                                              __int_as_float(e.x & 3));
+        }
+#pragma unroll
+        for (int q = 0; q < NP; q++) {
+            float p = pv[q].x, r = pv[q].y;
+            if constexpr (SENT && !std::is_same<S, float>::value) {
+                // narrow storage cannot hold -1e30: widen its empty marks (a
+                // slice without them has nothing to widen)
+                const float thr = empty_threshold<S>();
+                if (p <= thr) p = kSentinel;
+                if (r <= thr) r = kSentinel;
+            }
+            const float d = r - p;
+            // SENT: the extended value; else that minus (i - 1/2) d
+            const int i = q < ROUNDS ? lane : 64 + lane % (U > 0 ? U : 64);
+            const float gi = SENT ? (float)(w0v[q] + i - ga[q]) : (float)(w0v[q] - ga[q]) + 0.5f;
+            lds.pairs[slot[q]] = make_float2(fmaf(gi, d, p), d);
+        }
+        __syncthreads();
+        if (!live) continue;
+        // the voxels this thread updates, loaded beside the last chunk's
+        // sums (the WBP grid is written, not updated)
+        if (!WBP && c0 + CH >= n_list) {
+            int zo = z0;
+            asm volatile("" : "+s"(zo));   // the row offsets are formed here, not kept in registers
+#pragma unroll
+            for (int k = 0; k < TZ; k++)
+                vold[k] = ldb<float>(vres, xc * (int)sizeof(float), min(zo + k, vol_z - 1) * row_bytes);
+        }
+        // ---- accumulate ----
+        const char* pairs = (const char*)lds.pairs;
+        float4 next = lds.ent[wave][0];
+        float cm = 8388608.0f;
+        for (int j = 0; j < nc;) {
+            float4 e;
+            int cls;
+            // the tilts that every voxel uses run in a loop of their own: as
+            // one branch of a common loop, all sums were copied after a tilt
+            for (;;) {
+                e = next;
+                next = lds.ent[wave][j + 1];
+                cls = __builtin_amdgcn_readfirstlane(__float_as_int(e.w));
+                if (SENT || cls != 1) break;
+                full_cnt += 1;
+                const float v0 = fmaf(xf, e.y, e.x);
+                bp_full8<0>(pairs, e.z, v0, cm, acc);
+                if constexpr (TZ > 8) bp_full8<8>(pairs, e.z, v0, cm, acc);
+                cm += (float)WIN;
+                if (++j >= nc) break;
+            }
+            if (j >= nc) break;
+            const float ss = e.z;
+            const float v0 = fmaf(xf, e.y, e.x);
+            const int jp = j++;
+            const float cp = cm;
+            cm += (float)WIN;
+            if (cls == 0) continue;
+            partial = true;
+            const cptr<int2> lh = as_cptr(A->lohi) +
+                                  (size_t)ldc(as_cptr(A->list) + c0 + jp).tilt * A->lohi_stride + z0;
+#pragma unroll
+            for (int k0 = 0; k0 < TZ; k0 += 8) {
+                const BpRows8 rows = ldc((cptr<BpRows8>)(lh + k0));
+#pragma unroll
+                for (int m = 0; m < 8; m++) {
+                    const int k = k0 + m;
+                    const float v = fmaf((float)k, ss, v0);
+                    float val;
+                    bool in = (x >= rows.r[m].x) & (x <= rows.r[m].y);
+                    if (SENT) {
+                        const float u = v + 0.5f;
+                        const float2 pr = lds.pairs[jp * WIN + (int)u];
+                        val = fmaf(__builtin_amdgcn_fractf(u), pr.y, pr.x);
+                        in = in & !(val <= kEmpty);
+                    } else {
+                        const float2 pr = *(const float2*)(pairs + bp_addr(v, cp));
+                        val = fmaf(v, pr.y, pr.x);
+                    }
+                    acc[k] += in ? val : 0.0f;
+                    cnt[k / 2] += in ? (k % 2 ? 0x10000u : 1u) : 0u;
                 }
             }
         }
-        __syncthreads();
     }
-    if (WBP) {
-        // ---- mean over the tilts used, 0 when none (GBackProjWbp.cu:48-52) ----
+    if (!live || x >= vol_x) return;
+    const int n_rows = min(TZ, vol_z - z0);
+    const int voff = x * (int)sizeof(float);
+    bool wrote_sent = false;
+    // one row: its sum, the reciprocal of its count (with the relaxation)
+    auto write = [&](int k, float scale, bool any) {
+        const int so = (z0 + k) * row_bytes;
+        if (WBP) {
+            // mean over the tilts used, 0 when none (GBackProjWbp.cu:48-52)
+            stb(vres, any ? acc[k] * scale : 0.0f, voff, so);
+        } else {
+            // v = relax * sum / count + v, positivity, sentinel (GBackProj.cu:50-59)
+            float v = fmaf(acc[k], scale, vold[k]);
+            const bool empty = !(v > kEmpty);
+            v = empty ? kSentinel : (positivity ? fmaxf(v, 0.0f) : v);
+            if (any) {
+                stb(vres, v, voff, so);
+                wrote_sent |= empty;
+            }
+        }
+    };
+    // every voxel of a wave without partial tiles used the same tilts
+    const float one = (WBP ? 1.0f : relax) * __builtin_amdgcn_rcpf((float)full_cnt);
+    auto rows = [&](auto all) {
 #pragma unroll
         for (int k = 0; k < TZ; k++) {
-            const int z = z0 + k;
-            const int count = full_cnt + cnt[k];
-            const float v = count > 0 ? acc[k] * __builtin_amdgcn_rcpf((float)count) : 0.0f;
-            if (x < vol_x && z < vol_z) stb(vres, v, x * (int)sizeof(float), z * row_bytes);
+            if (!decltype(all)::value && k >= n_rows) break;
+            if (!partial) {
+                write(k, one, full_cnt > 0);
+            } else {
+                const int count = full_cnt + (int)((cnt[k / 2] >> (k % 2 * 16)) & 0xffffu);
+                write(k, (WBP ? 1.0f : relax) * __builtin_amdgcn_rcpf((float)count), count > 0);
+            }
         }
-        return;
-    }
-    // ---- v = relax * sum / count + v, positivity, sentinel (GBackProj.cu:50-59) ----
-    bool wrote_sent = false;
-#pragma unroll
-    for (int k = 0; k < TZ; k++) {
-        const int z = z0 + k;
-        const int count = full_cnt + cnt[k];
-        float v = relax * acc[k] * __builtin_amdgcn_rcpf((float)count) + vold[k];
-        const bool empty = !(v > kEmpty);
-        v = empty ? kSentinel : (positivity ? fmaxf(v, 0.0f) : v);
-        if (x < vol_x && z < vol_z && count > 0) {
-            stb(vres, v, x * (int)sizeof(float), z * row_bytes);
-            wrote_sent |= empty;
-        }
-    }
-    if (wrote_sent) atomicOr(vflag + y, 1);
+    };
+    if (!WBP && !partial && full_cnt == 0) return;
+    if (!partial && n_rows == TZ) rows(std::true_type{});
+    else rows(std::false_type{});
+    if (!WBP && wrote_sent) atomicOr(A->vflag + y, 1);
 }
 
 template <typename S, int TZ, int CH, bool WBP = false>
-__device__ __forceinline__ void bp_tile(cptr<BpArgs> A, float2 (&pairs)[CH][bp_win(TZ)],
-                                        int xt, int zt, int y)
+__device__ __forceinline__ void bp_tile(cptr<BpArgs> A, BpLds<TZ, CH, WBP>& lds, int xt, int zt,
+                                        int y)
 {
     const cptr<int> sflag = as_cptr(A->sflag);
     if (sflag != nullptr && sflag[y] != 0)
-        bp_tile_body<S, TZ, CH, WBP, true>(A, pairs, xt, zt, y);
+        bp_tile_body<S, TZ, CH, WBP, true>(A, lds, xt, zt, y);
     else
-        bp_tile_body<S, TZ, CH, WBP, false>(A, pairs, xt, zt, y);
+        bp_tile_body<S, TZ, CH, WBP, false>(A, lds, xt, zt, y);
 }
 
+// n_y > 0: grid (8 x-tiles, z-tiles, slices / 8), n_y slices.  Workgroups go
+// to the eight XCDs in turn, so all tiles of a slice run on one XCD, whose L2
+// holds the slice's sinogram.  n_y = 0: grid (x-tiles, z-tiles, slices), for
+// few slices, whose tiles spread over the XCDs (bp_grid).
 template <typename S, int TZ, int CH>
-__global__ __launch_bounds__(BP_TX) void k_back_proj(const BpArgs* __restrict__ a)
+__global__ __launch_bounds__(BP_THREADS, 5) void k_back_proj(const BpArgs* __restrict__ a, int n_y)
 {
-    __shared__ float2 pairs[CH][bp_win(TZ)];
-    bp_tile<S, TZ, CH>(as_cptr(a), pairs, blockIdx.x, blockIdx.y, blockIdx.z);
+    __shared__ BpLds<TZ, CH, false> lds;
+    const int per = n_y > 0 ? XCDS : 1;
+    const int y = blockIdx.z * per + blockIdx.x % per;
+    if (n_y > 0 && y >= n_y) return;
+    bp_tile<S, TZ, CH>(as_cptr(a), lds, blockIdx.x / per, blockIdx.y, y);
 }
 
 // WBP back-projection onto the 2x grid (Recon/GBackProjWbp.cu:14-53): the
 // same tile machinery, coordinate u = (fx cos + fz sin)/2 + P/2 + 1/2, the
 // mean written to the grid buffer.
-template <typename S>
-__global__ __launch_bounds__(BP_TX) void k_wbp_grid_bp(const BpArgs* __restrict__ a)
+template <typename S, int TZ>
+__global__ __launch_bounds__(BP_THREADS, 6) void k_wbp_grid_bp(const BpArgs* __restrict__ a, int n_y)
 {
-    __shared__ float2 pairs[BP_CHUNK][bp_win(BP_TZ)];
-    bp_tile<S, BP_TZ, BP_CHUNK, true>(as_cptr(a), pairs, blockIdx.x, blockIdx.y, blockIdx.z);
+    __shared__ BpLds<TZ, BP_WBP_CHUNK, true> lds;
+    const int per = n_y > 0 ? XCDS : 1;
+    const int y = blockIdx.z * per + blockIdx.x % per;
+    if (n_y > 0 && y >= n_y) return;
+    bp_tile<S, TZ, BP_WBP_CHUNK, true>(as_cptr(a), lds, blockIdx.x / per, blockIdx.y, y);
 }
 
 // Back-projection of many series in persistent launches: blocks take
@@ -433,11 +565,11 @@ __global__ __launch_bounds__(BP_TX) void k_wbp_grid_bp(const BpArgs* __restrict_
 // per stage, 1: 16 x 8, 2: 8 x 16, 3: 8 x 8), so each shape's kernel holds
 // only its own code and registers, as the per-series kernels do.
 template <typename S, int SHAPE>
-__global__ __launch_bounds__(BP_TX) void k_back_proj_batch(const BpItem* __restrict__ e, int n_e,
+__global__ __launch_bounds__(BP_THREADS) void k_back_proj_batch(const BpItem* __restrict__ e, int n_e,
                                                            int total, int* __restrict__ counter)
 {
     constexpr int TZ = (SHAPE & 2) ? 8 : 16, CH = (SHAPE & 1) ? 8 : 16;
-    __shared__ float2 pairs[CH][bp_win(TZ)];
+    __shared__ BpLds<TZ, CH, false> lds;
     const cptr<BpItem> E = as_cptr(e);
     int s = 0;
     for (int it = publish_item(claim_item(counter)); it < total;) {
@@ -451,7 +583,8 @@ __global__ __launch_bounds__(BP_TX) void k_back_proj_batch(const BpItem* __restr
             const int r = q * BP_ITEM_TILES + g;
             if (r >= nt) break;
             const int zt = r / nx, xt = r - zt * nx;
-            bp_tile<S, TZ, CH>(&E[s].a, pairs, xt, zt, y);
+            if (g > 0) __syncthreads();
+            bp_tile<S, TZ, CH>(&E[s].a, lds, xt, zt, y);
         }
         it = publish_item(ahead);
     }
@@ -618,25 +751,23 @@ void launch_weight_sart(const Plan& p, const float* in, hipStream_t s)
     else launch_weight_t<float>(p, in, s);
 }
 
-BpArgs bp_args(const Plan& p, const void* sino, int rows, const TiltRow* list, int n_list,
-               float relax, bool check_sent)
+BpArgs bp_args(const Plan& p, const void* sino, int rows, int first, int n_list, float relax,
+               bool check_sent)
 {
     BpArgs a{};
     a.sino = sino;
     a.rows_per_slice = rows;
     a.stride = p.sino_stride;
     a.proj = p.proj;
-    a.list = list;
+    a.list = p.d_lists + first;
     a.n_list = n_list;
-    a.cs = p.d_cs;
     a.lohi = p.d_bp_lohi;
-    a.tiles = p.d_bp_tiles;
-    a.n_ztiles = (p.vol_z + p.bp_tz - 1) / p.bp_tz;
+    a.lohi_stride = bp_zpad(p.vol_z);
+    a.n_ztiles = bp_ztiles(p.vol_z, p.bp_tz);
     a.n_xtiles = (p.vol_x + BP_TX - 1) / BP_TX;
+    a.tiles = p.d_bp_tiles + (size_t)a.n_ztiles * BP_WAVES * a.n_xtiles * first;
     a.relax = relax;
     a.positivity = p.positivity;
-    a.scale = 1.0f;
-    a.offset = (float)(p.proj / 2.0);
     a.sflag = check_sent ? p.d_sflag : nullptr;
     a.vol = p.d_vol;
     a.vol_x = p.vol_x;
@@ -645,12 +776,25 @@ BpArgs bp_args(const Plan& p, const void* sino, int rows, const TiltRow* list, i
     return a;
 }
 
+// Grid of a back-projection; *n_y: its argument.
+static dim3 bp_grid(int vol_x, int vol_y, int vol_z, int tz, int* n_y)
+{
+    const int nxt = (vol_x + BP_TX - 1) / BP_TX, nzt = bp_ztiles(vol_z, tz);
+    if (vol_y < BP_XCD_SLICES) {
+        *n_y = 0;
+        return dim3(nxt, nzt, vol_y);
+    }
+    *n_y = vol_y;
+    return dim3(XCDS * nxt, nzt, (vol_y + XCDS - 1) / XCDS);
+}
+
 template <typename S, int TZ, int CH>
 static void launch_bp_v(const Plan& p, int step, hipStream_t s)
 {
-    const int nxt = (p.vol_x + BP_TX - 1) / BP_TX, nzt = (p.vol_z + TZ - 1) / TZ;
-    hipLaunchKernelGGL((k_back_proj<S, TZ, CH>), dim3(nxt, nzt, p.vol_y), dim3(BP_TX), 0, s,
-                       p.d_bp_args + step);
+    int n_y = 0;
+    const dim3 grid = bp_grid(p.vol_x, p.vol_y, p.vol_z, TZ, &n_y);
+    hipLaunchKernelGGL((k_back_proj<S, TZ, CH>), grid, dim3(BP_THREADS), 0, s, p.d_bp_args + step,
+                       n_y);
 }
 
 // Back-projection tile shapes the autotuner chooses from: z rows per thread
@@ -671,14 +815,23 @@ void launch_bp(const Plan& p, int step, hipStream_t s)
     else launch_bp_t<float>(p, step, s);
 }
 
+template <typename S>
+static void launch_wbp_bp_t(const Plan& p, const BpArgs* a, int ny, hipStream_t s)
+{
+    int n_y = 0;
+    const dim3 grid = bp_grid(2 * p.vol_x, ny, 2 * p.vol_z, p.bp_tz, &n_y);
+    if (p.bp_tz == 8)
+        hipLaunchKernelGGL((k_wbp_grid_bp<S, 8>), grid, dim3(BP_THREADS), 0, s, a, n_y);
+    else
+        hipLaunchKernelGGL((k_wbp_grid_bp<S, 16>), grid, dim3(BP_THREADS), 0, s, a, n_y);
+}
+
 void launch_wbp_bp(const Plan& p, int slab, int ny, hipStream_t s)
 {
-    const int nxt = (2 * p.vol_x + BP_TX - 1) / BP_TX, nzt = (2 * p.vol_z + BP_TZ - 1) / BP_TZ;
-    dim3 grid(nxt, nzt, ny);
     const BpArgs* a = p.d_bp_args + slab;
-    if (p.storage == ATR_STORAGE_F16) hipLaunchKernelGGL(k_wbp_grid_bp<_Float16>, grid, dim3(BP_TX), 0, s, a);
-    else if (p.storage == ATR_STORAGE_BF16) hipLaunchKernelGGL(k_wbp_grid_bp<bf16_t>, grid, dim3(BP_TX), 0, s, a);
-    else hipLaunchKernelGGL(k_wbp_grid_bp<float>, grid, dim3(BP_TX), 0, s, a);
+    if (p.storage == ATR_STORAGE_F16) launch_wbp_bp_t<_Float16>(p, a, ny, s);
+    else if (p.storage == ATR_STORAGE_BF16) launch_wbp_bp_t<bf16_t>(p, a, ny, s);
+    else launch_wbp_bp_t<float>(p, a, ny, s);
 }
 
 std::vector<BpLaunch> lay_out_bp(const std::vector<QueueEntry<BpItem>>& ent, BpItem* out)
@@ -705,10 +858,10 @@ static int bp_batch_v(const BpLaunch* l, const BpItem* items, int* counter, int 
     if (!items) {
         int nb = 0;
         const hipError_t e =
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_back_proj_batch<S, SHAPE>, BP_TX, 0);
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_back_proj_batch<S, SHAPE>, BP_THREADS, 0);
         return (e == hipSuccess && nb > 0) ? nb : 1;
     }
-    hipLaunchKernelGGL((k_back_proj_batch<S, SHAPE>), dim3(grid), dim3(BP_TX), 0, s, items,
+    hipLaunchKernelGGL((k_back_proj_batch<S, SHAPE>), dim3(grid), dim3(BP_THREADS), 0, s, items,
                        l->n_entries, l->total, counter);
     return 0;
 }

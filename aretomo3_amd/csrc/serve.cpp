@@ -429,7 +429,7 @@ static atr_status run_round(atr_server* s)
         const int n_all = (int)p.all_tilts.size();
         if (r.step == 0) {
             BpItem e{};
-            e.a = bp_args(p, p.d_sino, p.n, p.d_lists, n_all, 1.0f, true);
+            e.a = bp_args(p, p.d_sino, p.n, 0, n_all, 1.0f, true);
             e.n_items_y = bp_items_per_slice(e.a);
             e.shape = bp_shape(p.bp_tz, p.bp_chunk);
             bent.push_back({e, p.vol_y * e.n_items_y, (double)n_all * p.bp_tz});
@@ -444,7 +444,7 @@ static atr_status run_round(atr_server* s)
                             (double)p.vol_x * p.vol_z * std::min(f.a.group, f1 - f0)});
             if (b1 > b0) {
                 BpItem e{};
-                e.a = bp_args(p, p.d_diff, p.max_subset, p.d_lists + n_all + b0, b1 - b0, p.relax,
+                e.a = bp_args(p, p.d_diff, p.max_subset, n_all + b0, b1 - b0, p.relax,
                               false);
                 e.n_items_y = bp_items_per_slice(e.a);
                 e.shape = bp_shape(p.bp_tz, p.bp_chunk);

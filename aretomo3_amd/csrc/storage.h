@@ -111,6 +111,18 @@ __device__ __forceinline__ float ldb<bf16_t>(__amdgpu_buffer_rsrc_t r, int voff,
 {
     return __uint_as_float((uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0) << 16);
 }
+// Two consecutive elements.
+template <typename S>
+__device__ __forceinline__ float2 ldb2(__amdgpu_buffer_rsrc_t r, int voff, int soff)
+{
+    return make_float2(ldb<S>(r, voff, soff), ldb<S>(r, voff + (int)sizeof(S), soff));
+}
+template <>
+__device__ __forceinline__ float2 ldb2<float>(__amdgpu_buffer_rsrc_t r, int voff, int soff)
+{
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+    return make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
+}
 __device__ __forceinline__ void stb(__amdgpu_buffer_rsrc_t r, float v, int voff, int soff)
 {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, voff, soff, 0);
