@@ -371,12 +371,14 @@ constexpr int REPROJ_MAX_TILTS = 10;
 struct ReprojArgs {
     int proj_x, proj_y, vol_x, vol_z;
     int first, n_range, ray;
+    int seg, width;            // samples per staged segment, columns staged (set at launch)
     float min_count;
     double cos_t[REPROJ_MAX_TILTS], sin_t[REPROJ_MAX_TILTS], weight[REPROJ_MAX_TILTS];
+    double cos_w[REPROJ_MAX_TILTS];   // cos_t * weight
+    double total, inv_total;          // sum of the weights
     double ray_cos, ray_sin;
 };
-void launch_reproj(const ReprojArgs& a, const float* projs, float* vol_slab, int slab_rows,
-                   float* out, hipStream_t s);
+void launch_reproj(const ReprojArgs& args, const float* projs, float* out, hipStream_t s);
 
 // What the weighting / filter kernels read: the binned images, the
 // pre-stage output (with the random fill), or the caller's input.
