@@ -242,12 +242,13 @@ static size_t plan_bytes_estimate(const Plan& p)
         b += n * p.vol_z * 8 + n * p.proj * 8 + (size_t)p.vol_x * p.vol_z * 4;
         b += n * (size_t)(p.vol_z * 2.5 + 16) * 16;  // FP sample tables (bounded by 60 deg)
         // back-projection tiles: every tilt is in the initial list and in a subset's
-        b += 2 * n * (size_t)bp_ztiles(p.vol_z, 8) * BP_WAVES * ((p.vol_x + BP_TX - 1) / BP_TX) * sizeof(int2);
+        const int kind = bp_kind_of(p.storage);
+        b += 2 * n * (size_t)bp_ztiles(p.vol_z, 8, kind) * bp_xtiles(p.vol_x, kind) * BP_WAVES * sizeof(int2);
     } else {
         b += (size_t)p.wbp_slab * 3 * p.vol_z * (p.vol_x / 2 + 1) * sizeof(float2);
         b += (size_t)p.wbp_slab * 4 * p.vol_z * p.vol_x * sizeof(float);
         b += n * 2 * p.vol_z * 8 + n * 16;
-        b += n * (size_t)bp_ztiles(2 * p.vol_z, 8) * BP_WAVES * ((2 * p.vol_x + BP_TX - 1) / BP_TX) * sizeof(int2);
+        b += n * (size_t)bp_ztiles(2 * p.vol_z, 8, BP_GRID) * bp_xtiles(2 * p.vol_x, BP_GRID) * BP_WAVES * sizeof(int2);
     }
     return b;
 }
@@ -281,7 +282,7 @@ static atr_status sart_tables_host(Plan& p, int tz, int chunk, int bz, int pf)
     std::vector<int> ends(1, (int)p.all_tilts.size());
     for (int sb = 0; sb < p.n_subsets; sb++) ends.push_back(ends[0] + p.subset_off[sb + 1]);
     build_bp_tiles(lists, ends, g.cos_sin, g.bp_lohi, p.vol_x, p.vol_z, 1.0, p.proj / 2.0, tz,
-                   g.bp_tiles);
+                   bp_kind_of(p.storage), g.bp_tiles);
     if (!build_fp_tables(g.cos_sin, p.n, p.vol_x, p.vol_z, p.proj, bz, g))
         return fail(ATR_ERR_INVALID_ARG, "SART needs every tilt in (-90, 90) degrees");
     std::vector<int>& sched = p.host.sched;
@@ -396,7 +397,7 @@ static atr_status plan_host(Plan& p)
         fill_table(d.fill_seed ^ 0x5A5A5A5A5A5A5A5Aull, p.vol_x * p.vol_z, h.fill_vol);
         // back-projection tiles: a stage as large as a subset of up to 8 tilts
         // (2-5 % less than 16 tilts a stage at 5 to 6 tilts, 3 % more at 12)
-        p.bp_tz = bp_default_tz(p.vol_x, p.vol_y, p.vol_z);
+        p.bp_tz = bp_default_tz(p.vol_x, p.vol_y, p.vol_z, bp_kind_of(p.storage));
         p.bp_chunk = p.max_subset <= 8 ? 8 : 16;
         // default forward-projector staging: register prefetch where it is
         // built (VolX 1024, 2048: measured faster at the full band height),
@@ -408,10 +409,10 @@ static atr_status plan_host(Plan& p)
     build_wbp_intervals(g.cos_sin, p.n, p.vol_x, p.vol_z, p.proj, g.wbp_lohi);
     // 2x-grid back-projection: tile windows/classes (excluded tilts are left
     // out of the list, GBackProjWbp.cu:31)
-    p.bp_tz = bp_default_tz(2 * p.vol_x, std::min(p.wbp_slab, p.vol_y), 2 * p.vol_z);
+    p.bp_tz = bp_default_tz(2 * p.vol_x, std::min(p.wbp_slab, p.vol_y), 2 * p.vol_z, BP_GRID);
     h.lists = bp_list(g.cos_sin, p.all_tilts, 0.5f);
     build_bp_tiles(h.lists, {(int)p.all_tilts.size()}, g.cos_sin, g.wbp_lohi, 2 * p.vol_x,
-                   2 * p.vol_z, 0.5, (double)(p.proj / 2) + 0.5, p.bp_tz, h.wbp_tiles);
+                   2 * p.vol_z, 0.5, (double)(p.proj / 2) + 0.5, p.bp_tz, BP_GRID, h.wbp_tiles);
     h.lists.resize(h.lists.size() + BP_PAD);
     h.filter = ramp_filter(p.proj);
     make_fft(p.proj, p.fft_proj);
@@ -494,8 +495,8 @@ static atr_status plan_device(Plan& p)
             a.lohi = p.d_wbp_lohi;
             a.lohi_stride = bp_zpad(2 * p.vol_z);
             a.tiles = p.d_wbp_tiles;
-            a.n_ztiles = bp_ztiles(2 * p.vol_z, p.bp_tz);
-            a.n_xtiles = (2 * p.vol_x + BP_TX - 1) / BP_TX;
+            a.n_ztiles = bp_ztiles(2 * p.vol_z, p.bp_tz, BP_GRID);
+            a.n_xtiles = bp_xtiles(2 * p.vol_x, BP_GRID);
             a.relax = 1.0f;
             a.positivity = 0;
             a.sflag = p.d_sflag + y0;

@@ -19,8 +19,11 @@ constexpr float kEmpty = -1e10f;
 constexpr float kSentinel = -1e30f;
 
 // ---- tile shapes ---------------------------------------------------------
-// Back-projection: a workgroup of BP_WAVES waves owns BP_TX x (BP_WAVES tz)
-// voxels of one slice; lane = x, each thread walks tz rows of z.
+// Back-projection: a workgroup of BP_WAVES waves owns a tile of one slice;
+// lane = x, each thread walks tz rows of z.  Square tiles (SART) and those of
+// the WBP's 2x grid are BP_TX x (BP_WAVES tz) voxels, wide tiles (SART with BF16
+// storage) (BP_WAVES BP_TX) x tz.
+enum { BP_SQUARE = 0, BP_GRID = 1, BP_WIDE = 2 };
 constexpr int BP_TX = 64;
 constexpr int BP_WAVES = 4;
 constexpr int BP_THREADS = 64 * BP_WAVES;
@@ -30,19 +33,35 @@ constexpr int XCDS = 8;                      // workgroups go to the XCDs in tur
 // reconstruction at 475 and 1024 slices, even at 256 and 300, 3 % slower at 64
 // and 96, where the XCDs' shares are uneven).
 constexpr int BP_XCD_SLICES = 256;
-// Staged pairs per tilt, at least one for each lane: the tile spans at most
-// sqrt(63^2 + (4 tz - 1)^2) samples (half that on the WBP's 2x grid);
-// build_bp_tiles leaves 3 before its smallest coordinate, and 2 follow the
-// largest.
-constexpr int bp_win(int tz, bool wbp) { return wbp ? 64 : tz == 16 ? 96 : 80; }
+inline int bp_kind_of(int storage) { return storage == ATR_STORAGE_BF16 ? BP_WIDE : BP_SQUARE; }
+// waves of a tile side by side in x
+constexpr int bp_wx(int kind) { return kind == BP_WIDE ? BP_WAVES : 1; }
+// Staged pairs per tilt, at least one for each lane: a square tile spans at
+// most sqrt(63^2 + (4 tz - 1)^2) samples (half that on the WBP's 2x grid), a
+// wide one 255 + tz; build_bp_tiles leaves 3 before its smallest coordinate,
+// and 2 follow the largest.
+constexpr int bp_win(int tz, int kind)
+{
+    return kind == BP_GRID ? 64 : kind == BP_WIDE ? 288 : tz == 16 ? 96 : 80;
+}
 // rows per tilt of an interval table: whole tiles of either height
 inline int bp_zpad(int vol_z) { return (vol_z + 63) / 64 * 64; }
-inline int bp_ztiles(int vol_z, int tz) { return (vol_z + BP_WAVES * tz - 1) / (BP_WAVES * tz); }
+inline int bp_ztiles(int vol_z, int tz, int kind)
+{
+    const int rows = BP_WAVES / bp_wx(kind) * tz;
+    return (vol_z + rows - 1) / rows;
+}
+inline int bp_xtiles(int vol_x, int kind)
+{
+    const int cols = bp_wx(kind) * BP_TX;
+    return (vol_x + cols - 1) / cols;
+}
 // Rows per thread unless tuned: 16, or 8 where 16 would leave fewer than four
 // workgroups per CU (few slices).
-inline int bp_default_tz(int vol_x, int vol_y, int vol_z)
+inline int bp_default_tz(int vol_x, int vol_y, int vol_z, int kind)
 {
-    const long tiles = (long)((vol_x + BP_TX - 1) / BP_TX) * bp_ztiles(vol_z, 16) * vol_y;
+    if (kind == BP_WIDE) return 16;
+    const long tiles = (long)bp_xtiles(vol_x, kind) * bp_ztiles(vol_z, 16, kind) * vol_y;
     return tiles < 1024 ? 8 : 16;
 }
 // Forward projection: a workgroup of FP_THREADS owns one slice and a group of
@@ -109,9 +128,10 @@ constexpr int BP_PAD = 32;
 struct Geometry {
     std::vector<float> cos_sin;        // [2N] float, as CTomoBase.cpp:55-65
     std::vector<int2> bp_lohi;         // [N][bp_zpad(VolZ)] x-interval of GBackProj inclusion
-    // per list of n tilts: [4 ztiles][xtiles][n], one entry per wave of a
-    // tile: {4 window start + class (0 empty / 1 full / 2 partial), FP32 bits
-    // of u - start - 1/2 at the wave's first voxel}
+    // per list of n tilts: [waves in z][waves in x][n], one entry per wave of
+    // a tile: {4 window start + class (0 empty / 1 full / 2 partial), FP32 bits
+    // of u - start - 1/2 at the wave's first voxel (wide tiles: u - start at
+    // the tile's)}
     std::vector<int2> bp_tiles;
     std::vector<int2> wbp_lohi;        // [N][bp_zpad(2VolZ)] x2-interval of GBackProjWbp inclusion
     std::vector<int2> fp_range;        // [N][P] first valid sample and count of each ray
@@ -258,7 +278,7 @@ struct BpArgs {
     int n_list;
     int lohi_stride;
     const int2* lohi;          // [N][lohi_stride]
-    const int2* tiles;         // [4 ztiles][xtiles][n_list], Geometry::bp_tiles
+    const int2* tiles;         // [waves in z][waves in x][n_list], Geometry::bp_tiles
     int n_ztiles, n_xtiles;
     float relax;
     int positivity;
@@ -426,7 +446,8 @@ std::vector<BpTilt> bp_list(const std::vector<float>& cs, const std::vector<Tilt
 // lists: tilts of every list one after another, ends: where each list ends
 void build_bp_tiles(const std::vector<BpTilt>& lists, const std::vector<int>& ends,
                     const std::vector<float>& cs, const std::vector<int2>& lohi, int vol_x,
-                    int vol_z, double scale, double offset, int tz, std::vector<int2>& tiles);
+                    int vol_z, double scale, double offset, int tz, int kind,
+                    std::vector<int2>& tiles);
 void build_wbp_intervals(const std::vector<float>& cs, int n, int vol_x, int vol_z, int proj,
                          std::vector<int2>& lohi);
 bool build_fp_tables(const std::vector<float>& cs, int n, int vol_x, int vol_z, int proj,

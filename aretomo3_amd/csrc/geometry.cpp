@@ -130,23 +130,25 @@ void build_bp_intervals(const std::vector<float>& cs, int n, int vol_x, int vol_
     });
 }
 
-// Back-projection tiles of BP_TX x (BP_WAVES tz) voxels: per wave (tz rows),
-// x-tile and tilt, the start w0 of the row window that the tile stages (the
-// same for its waves), the class of the wave's voxels (1 = every one uses the
-// tilt, 0 = none does, 2 = some do; 0 below the volume) and the coordinate of
-// its first one.  The grid coordinate is u = scale (fx cos + fz sin) + offset
-// (SART: scale 1, offset P/2; the WBP 2x grid: scale 1/2, offset P/2 + 1/2).
-// w0 = floor(min u over the tile corners) - 3 in FP64; the kernel's FP32
-// coordinates relative to w0 then stay in [2, window - 2].  The second field
-// holds the FP32 bits of u - w0 - 1/2 at the wave's first voxel, formed in
-// FP64: the kernel adds (x - x0) scale cos and k scale sin to it in FP32, and
-// rounding the sum to the nearest integer gives the cell.
+// Back-projection tiles: per wave (tz rows x BP_TX columns) and tilt, the start
+// w0 of the row window that the tile stages (the same for its waves), the class
+// of the wave's voxels (1 = every one uses the tilt, 0 = none does, 2 = some
+// do; 0 outside the volume) and a first coordinate.  The grid coordinate is
+// u = scale (fx cos + fz sin) + offset (SART: scale 1, offset P/2; the WBP 2x
+// grid: scale 1/2, offset P/2 + 1/2).  w0 = floor(min u over the tile corners)
+// - 3 in FP64; the kernel's FP32 coordinates relative to w0 then stay in [2,
+// window - 2].  The second field holds the FP32 bits of u - w0 - 1/2 at the
+// wave's first voxel (wide tiles: of u - w0 at the tile's), formed in FP64: the
+// kernel adds (x - x0) scale cos and k scale sin to it in FP32, and rounding
+// (wide tiles: truncating) the sum gives the cell.
 void build_bp_tiles(const std::vector<BpTilt>& lists, const std::vector<int>& ends,
                     const std::vector<float>& cs, const std::vector<int2>& lohi, int vol_x,
-                    int vol_z, double scale, double offset, int tz, std::vector<int2>& tiles)
+                    int vol_z, double scale, double offset, int tz, int kind,
+                    std::vector<int2>& tiles)
 {
-    const int nzt = bp_ztiles(vol_z, tz), nxt = (vol_x + BP_TX - 1) / BP_TX;
-    const size_t per = (size_t)nzt * BP_WAVES * nxt;
+    const int wx = bp_wx(kind), wz = BP_WAVES / wx;
+    const int nzt = bp_ztiles(vol_z, tz, kind), nxt = bp_xtiles(vol_x, kind);
+    const size_t per = (size_t)nzt * nxt * BP_WAVES;
     const int total = ends.back(), stride = bp_zpad(vol_z);
     tiles.assign(per * total + BP_PAD, int2{0, 0});
     parallel_tilts(total, [&](int l) {
@@ -157,10 +159,10 @@ void build_bp_tiles(const std::vector<BpTilt>& lists, const std::vector<int>& en
         const double c = cs[2 * t], s = cs[2 * t + 1];
         const int2* lh = lohi.data() + (size_t)t * stride;
         for (int zt = 0; zt < nzt; zt++) {
-            // per wave: the intervals' overlap and union over its rows
+            // per row of waves: the intervals' overlap and union over its rows
             int in_lo[BP_WAVES], in_hi[BP_WAVES], any_lo[BP_WAVES], any_hi[BP_WAVES];
-            for (int w = 0; w < BP_WAVES; w++) {
-                const int z0 = (zt * BP_WAVES + w) * tz, z1 = std::min(z0 + tz, vol_z);
+            for (int w = 0; w < wz; w++) {
+                const int z0 = (zt * wz + w) * tz, z1 = std::min(z0 + tz, vol_z);
                 in_lo[w] = 0, in_hi[w] = z0 < vol_z ? vol_x : -1;
                 any_lo[w] = vol_x, any_hi[w] = -1;
                 for (int z = z0; z < z1; z++) {
@@ -172,21 +174,25 @@ void build_bp_tiles(const std::vector<BpTilt>& lists, const std::vector<int>& en
                     }
                 }
             }
-            const int zt0 = zt * BP_WAVES * tz;
-            const double fz0 = zt0 - vol_z * 0.5, fz1 = fz0 + (BP_WAVES * tz - 1);
+            const int zt0 = zt * wz * tz;
+            const double fz0 = zt0 - vol_z * 0.5, fz1 = fz0 + (wz * tz - 1);
             const double sz = std::min(s * fz0, s * fz1);
             for (int xt = 0; xt < nxt; xt++) {
-                const int x0 = xt * BP_TX, x1 = std::min(x0 + BP_TX, vol_x) - 1;
+                const int x0 = xt * wx * BP_TX, x1 = std::min(x0 + wx * BP_TX, vol_x) - 1;
                 const double fx0 = x0 - vol_x * 0.5, fx1 = x1 - vol_x * 0.5;
                 const int w0 = (int)std::floor(offset + scale * (std::min(c * fx0, c * fx1) + sz)) - 3;
                 for (int w = 0; w < BP_WAVES; w++) {
-                    const int z0 = zt0 + w * tz;
-                    // (a tile between the rows' intervals counts as partial)
-                    const bool full = in_lo[w] <= x0 && in_hi[w] >= x1;
-                    const bool any = any_lo[w] <= x1 && any_hi[w] >= x0;
+                    const int xw = w % wx, zw = w / wx;
+                    const int xa = x0 + xw * BP_TX, xb = std::min(xa + BP_TX, vol_x) - 1;
+                    const int z0 = zt0 + zw * tz;
+                    // (columns between the rows' intervals count as partial)
+                    const bool full = xa <= xb && in_lo[zw] <= xa && in_hi[zw] >= xb;
+                    const bool any = xa <= xb && any_lo[zw] <= xb && any_hi[zw] >= xa;
                     const float u00 =
-                        (float)(scale * (c * fx0 + s * (z0 - vol_z * 0.5)) + offset - w0 - 0.5);
-                    out[((size_t)(zt * BP_WAVES + w) * nxt + xt) * len] =
+                        kind == BP_WIDE
+                            ? (float)(scale * (c * fx0 + s * fz0) + offset - w0)
+                            : (float)(scale * (c * fx0 + s * (z0 - vol_z * 0.5)) + offset - w0 - 0.5);
+                    out[((size_t)(zt * wz + zw) * (nxt * wx) + xt * wx + xw) * len] =
                         int2{4 * w0 + (full ? 1 : (any ? 2 : 0)), __builtin_bit_cast(int, u00)};
                 }
             }

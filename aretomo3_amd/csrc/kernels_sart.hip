@@ -221,6 +221,12 @@ __global__ __launch_bounds__(256) void k_weight(const float* __restrict__ in, si
 // its first voxel, cos, sin, class) is put into LDS with the rows and read
 // one tilt ahead, so no scalar-load latency stands between two tilts.
 //
+// BF16 storage runs SART on wide tiles (256 x TZ, waves side by side in x), with
+// coordinates rounded relative to the tile's first voxel, truncated and scaled
+// as they always were there: the differences are stored in BF16 after every
+// step, so a coordinate rounded otherwise, however little, moves some of them
+// by a whole unit of 2^-8, and single voxels by 1e-3 of the volume's rms.
+//
 // 1024^2 x 256, 12 to 13 tilts: 0.55 ms a launch (0.895 with 256 x 16 voxel
 // tiles, scalar operands and a conversion per update); 4.0 TB/s of the 4.9 a
 // large copy reaches.  WBP grid of 512^2 x 128, 41 tilts: 0.71 ms (1.29).  What
@@ -228,17 +234,22 @@ __global__ __launch_bounds__(256) void k_weight(const float* __restrict__ in, si
 // the 11.5 issue cycles of an update; 5 (WBP: 6) waves per SIMD hide the
 // staging loads and the barrier.
 // ------------------------------------------------------------------------
-template <int TZ, int CH, bool WBP>
+template <int TZ, int CH, int KIND>
 struct BpLds {
-    float2 pairs[CH * bp_win(TZ, WBP)];
-    // per wave and tilt: u - w0 - 1/2 at the wave's first voxel, scaled cos
-    // and sin, class; one spare entry, read ahead of the last tilt
+    float2 pairs[CH * bp_win(TZ, KIND)];
+    // per wave and tilt: u - w0 - 1/2 at the wave's first voxel (wide: u - w0
+    // at the tile's), scaled cos and sin, class; one spare entry, read ahead of
+    // the last tilt
     float4 ent[BP_WAVES][CH + 1];
 };
 
 // Byte address of the pair that v (plus the 2^23 of cm) falls into.
+// Wide tiles: v is the coordinate itself, truncated, and cm carries the bits of
+// the window's byte offset.
+template <bool WIDE>
 __device__ __forceinline__ unsigned bp_addr(float v, float cm)
 {
+    if constexpr (WIDE) return 8 * (int)v + __float_as_int(cm);
     unsigned a;
     asm("v_lshlrev_b16 %0, 3, %1" : "=v"(a) : "v"(v + cm));
     return a;
@@ -260,7 +271,7 @@ __device__ __forceinline__ float bp_coord(float ss, float v0)
 
 // Rows K0 .. K0 + 7 of a tilt that every voxel uses: the eight LDS reads go
 // out before the first value is needed.
-template <int K0, int TZ>
+template <int K0, int TZ, bool WIDE>
 __device__ __forceinline__ void bp_full8(const char* pairs, float ss, float v0, float cm,
                                          float (&acc)[TZ])
 {
@@ -275,7 +286,7 @@ __device__ __forceinline__ void bp_full8(const char* pairs, float ss, float v0, 
     v[6] = bp_coord<K0 + 6>(ss, v0);
     v[7] = bp_coord<K0 + 7>(ss, v0);
 #pragma unroll
-    for (int k = 0; k < 8; k++) pr[k] = *(const float2*)(pairs + bp_addr(v[k], cm));
+    for (int k = 0; k < 8; k++) pr[k] = *(const float2*)(pairs + bp_addr<WIDE>(v[k], cm));
 #pragma unroll
     for (int k = 0; k < 8; k++) acc[K0 + k] += fmaf(v[k], pr[k].y, pr[k].x);
 }
@@ -290,21 +301,24 @@ struct BpRows8 {
 // SENT: the slice's sinogram rows may hold empty samples.  The staged pair is
 // then (q_i, d_i) and the value q + fract(u) d, whose sentinel test must see
 // the exact -1e30 scale.
-template <typename S, int TZ, int CH, bool WBP, bool SENT>
-__device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>& lds, int xt,
+template <typename S, int TZ, int CH, int KIND, bool SENT>
+__device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, KIND>& lds, int xt,
                                              int zt, int y)
 {
-    constexpr int WIN = bp_win(TZ, WBP);
+    constexpr bool WBP = KIND == BP_GRID, WIDE = KIND == BP_WIDE;
+    constexpr int WIN = bp_win(TZ, KIND);
+    // waves side by side in x and in z
+    constexpr int WX = bp_wx(KIND), WZ = BP_WAVES / WX;
     const int rows_per_slice = A->rows_per_slice, stride = A->stride, proj = A->proj;
-    const int n_list = A->n_list, n_xtiles = A->n_xtiles;
+    const int n_list = A->n_list;
     const int vol_x = A->vol_x, vol_z = A->vol_z;
     const float relax = A->relax;
     const int positivity = A->positivity;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int x0 = xt * BP_TX, zq = zt * BP_WAVES + wave, z0 = zq * TZ;
-    const bool live = z0 < vol_z;
-    const int x = x0 + lane;
+    const int xq = xt * WX + wave % WX, zq = zt * WZ + wave / WX, z0 = zq * TZ;
+    const bool live = z0 < vol_z && xq * BP_TX < vol_x;
+    const int x = xq * BP_TX + lane;
     const int xc = min(x, vol_x - 1);
     // the slice and its sinogram rows as buffers: a row offset is a scalar, a
     // column the lane's fixed byte offset
@@ -317,7 +331,8 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
         buffer_of((const void*)base, (size_t)rows_per_slice * stride * sizeof(S));
     // window starts are those of the workgroup's tile (the same in the
     // entries of all its waves); coordinates and classes are the wave's
-    const gptr<const int2> etab = as_gptr(A->tiles) + ((size_t)zq * n_xtiles + xt) * n_list;
+    const size_t entries = ((size_t)zq * (A->n_xtiles * WX) + xq) * n_list;
+    const gptr<const int2> etab = as_gptr(A->tiles) + entries;
 
     float vold[TZ];
     float acc[TZ];
@@ -329,7 +344,7 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
     for (int k = 0; k < TZ / 2; k++) cnt[k] = 0;
     int full_cnt = 0;
     bool partial = false;
-    const float xf = (float)(xc - x0);   // offset from the tile's first voxel
+    const float xf = (float)(xc - xt * WX * BP_TX);   // offset from the tile's first voxel
 
     for (int c0 = 0; c0 < n_list; c0 += CH) {
         const int nc = min(CH, n_list - c0);
@@ -341,78 +356,84 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
         // the plain pair; at g = -1 it extrapolates, so a coordinate that FP32
         // rounding puts just below 0 still interpolates the first sample.
         // Pairs further out are only read by voxels the exact intervals
-        // exclude.  The first 64 pairs of a tilt take one wave instruction,
-        // the U others share one with those of GU - 1 more tilts.  Past the
-        // list's end the tables go on (into the next list, or their padding):
-        // what is staged for those slots is not read.  All loads are issued
-        // before a pair is formed, on every path alike. ----
-        constexpr int ROUNDS = CH / BP_WAVES;
-        constexpr int U = WIN > 64 ? WIN - 64 : 0, GU = U > 0 ? 64 / U : 1;
-        constexpr int UP = U > 0 ? (ROUNDS + GU - 1) / GU : 0, NP = ROUNDS + UP;
+        // exclude.  Each 64 pairs of a tilt take one wave instruction, the U
+        // others share one with those of GU - 1 more tilts.  Past the list's
+        // end the tables go on (into the next list, or their padding): what is
+        // staged for those slots is not read.  All loads are issued before a
+        // pair is formed, on every path alike (wide tiles, whose windows are
+        // longer: two tilts at a time). ----
+        constexpr int ROUNDS = CH / BP_WAVES, RND = WIDE ? 2 : ROUNDS;
+        constexpr int MF = WIN / 64, U = WIN % 64, GU = U > 0 ? 64 / U : 1;
+        constexpr int UP = U > 0 ? (RND + GU - 1) / GU : 0, NP = RND * MF + UP;
         struct WindowStarts {
-            int2 e[ROUNDS];
+            int2 e[RND];
         };
         struct Tilts {
-            BpTilt t[ROUNDS];
+            BpTilt t[RND];
         };
-        const int jw = wave * ROUNDS;
-        const WindowStarts ws =
-            ldc((cptr<WindowStarts>)(as_cptr(A->tiles) + ((size_t)zq * n_xtiles + xt) * n_list + c0 + jw));
-        const Tilts tl = ldc((cptr<Tilts>)(as_cptr(A->list) + c0 + jw));
-        float2 pv[NP];
-        int ga[NP], w0v[NP], slot[NP];
 #pragma unroll
-        for (int q = 0; q < NP; q++) {
-            int w0, voff, soff = 0;
-            if (q < ROUNDS) {
-                w0 = ws.e[q].x >> 2;
-                slot[q] = (jw + q) * WIN + lane;
-                ga[q] = min(max(w0 + lane, 0), proj - 2);
-                voff = ga[q] * (int)sizeof(S);
-                soff = tl.t[q].row * stride * (int)sizeof(S);
-            } else {
-                // lanes U s .. U s + U - 1: the upper pairs of tilt
-                // (q - ROUNDS) GU + s (the last one again past the wave's)
-                const int s = lane / (U > 0 ? U : 64), i = 64 + lane % (U > 0 ? U : 64);
-                int row = 0, r = 0;
-                w0 = 0;
+        for (int h = 0; h < ROUNDS; h += RND) {
+            const int jw = wave * ROUNDS + h;
+            const WindowStarts ws = ldc((cptr<WindowStarts>)(as_cptr(A->tiles) + entries + c0 + jw));
+            const Tilts tl = ldc((cptr<Tilts>)(as_cptr(A->list) + c0 + jw));
+            float2 pv[NP];
+            int ga[NP], w0v[NP], slot[NP];
 #pragma unroll
-                for (int h = 0; h < GU; h++) {
-                    const int qq = min((q - ROUNDS) * GU + h, ROUNDS - 1);
-                    if (h == 0 || s >= h) {
-                        w0 = ws.e[qq].x >> 2;
-                        row = tl.t[qq].row;
-                        r = qq;
+            for (int q = 0; q < NP; q++) {
+                int w0, voff, soff = 0;
+                if (q < RND * MF) {
+                    const int r = q / MF, i = lane + q % MF * 64;
+                    w0 = ws.e[r].x >> 2;
+                    slot[q] = (jw + r) * WIN + i;
+                    ga[q] = min(max(w0 + i, 0), proj - 2);
+                    voff = ga[q] * (int)sizeof(S);
+                    soff = tl.t[r].row * stride * (int)sizeof(S);
+                } else {
+                    // lanes U s .. U s + U - 1: the upper pairs of tilt
+                    // (q - RND MF) GU + s (the last one again past the wave's)
+                    const int s = lane / (U > 0 ? U : 64), i = MF * 64 + lane % (U > 0 ? U : 64);
+                    int row = 0, r = 0;
+                    w0 = 0;
+#pragma unroll
+                    for (int g = 0; g < GU; g++) {
+                        const int qq = min((q - RND * MF) * GU + g, RND - 1);
+                        if (g == 0 || s >= g) {
+                            w0 = ws.e[qq].x >> 2;
+                            row = tl.t[qq].row;
+                            r = qq;
+                        }
                     }
+                    slot[q] = (jw + r) * WIN + i;
+                    ga[q] = min(max(w0 + i, 0), proj - 2);
+                    voff = (row * stride + ga[q]) * (int)sizeof(S);
                 }
-                slot[q] = (jw + r) * WIN + i;
-                ga[q] = min(max(w0 + i, 0), proj - 2);
-                voff = (row * stride + ga[q]) * (int)sizeof(S);
+                w0v[q] = w0;
+                pv[q] = ldb2<S>(sres, voff, soff);
             }
-            w0v[q] = w0;
-            pv[q] = ldb2<S>(sres, voff, soff);
+#pragma unroll
+            for (int q = 0; q < NP; q++) {
+                float p = pv[q].x, r = pv[q].y;
+                if constexpr (SENT && !std::is_same<S, float>::value) {
+                    // narrow storage cannot hold -1e30: widen its empty marks
+                    // (a slice without them has nothing to widen)
+                    const float thr = empty_threshold<S>();
+                    if (p <= thr) p = kSentinel;
+                    if (r <= thr) r = kSentinel;
+                }
+                const float d = r - p;
+                // SENT: the extended value; else that minus (i - 1/2) d (wide:
+                // i d)
+                const int i = q < RND * MF ? lane + q % MF * 64 : MF * 64 + lane % (U > 0 ? U : 64);
+                const float gi = SENT ? (float)(w0v[q] + i - ga[q])
+                                      : (float)(w0v[q] - ga[q]) + (WIDE ? 0.0f : 0.5f);
+                lds.pairs[slot[q]] = make_float2(fmaf(gi, d, p), d);
+            }
         }
         if (lane < nc) {
             const int2 e = ldgo(etab + c0 + lane);
             const BpTilt bt = ldgo(as_gptr(A->list) + c0 + lane);
             lds.ent[wave][lane] = make_float4(__int_as_float(e.y), bt.c, bt.s,
                                               __int_as_float(e.x & 3));
-        }
-#pragma unroll
-        for (int q = 0; q < NP; q++) {
-            float p = pv[q].x, r = pv[q].y;
-            if constexpr (SENT && !std::is_same<S, float>::value) {
-                // narrow storage cannot hold -1e30: widen its empty marks (a
-                // slice without them has nothing to widen)
-                const float thr = empty_threshold<S>();
-                if (p <= thr) p = kSentinel;
-                if (r <= thr) r = kSentinel;
-            }
-            const float d = r - p;
-            // SENT: the extended value; else that minus (i - 1/2) d
-            const int i = q < ROUNDS ? lane : 64 + lane % (U > 0 ? U : 64);
-            const float gi = SENT ? (float)(w0v[q] + i - ga[q]) : (float)(w0v[q] - ga[q]) + 0.5f;
-            lds.pairs[slot[q]] = make_float2(fmaf(gi, d, p), d);
         }
         __syncthreads();
         if (!live) continue;
@@ -428,7 +449,12 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
         // ---- accumulate ----
         const char* pairs = (const char*)lds.pairs;
         float4 next = lds.ent[wave][0];
-        float cm = 8388608.0f;
+        // wide: the byte offset of the tilt's window, as an integer
+        float cm = WIDE ? 0.0f : 8388608.0f;
+        auto next_window = [&] {
+            if (WIDE) cm = __int_as_float(__float_as_int(cm) + WIN * 8);
+            else cm += (float)WIN;
+        };
         for (int j = 0; j < nc;) {
             float4 e;
             int cls;
@@ -441,9 +467,9 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
                 if (SENT || cls != 1) break;
                 full_cnt += 1;
                 const float v0 = fmaf(xf, e.y, e.x);
-                bp_full8<0>(pairs, e.z, v0, cm, acc);
-                if constexpr (TZ > 8) bp_full8<8>(pairs, e.z, v0, cm, acc);
-                cm += (float)WIN;
+                bp_full8<0, TZ, WIDE>(pairs, e.z, v0, cm, acc);
+                if constexpr (TZ > 8) bp_full8<8, TZ, WIDE>(pairs, e.z, v0, cm, acc);
+                next_window();
                 if (++j >= nc) break;
             }
             if (j >= nc) break;
@@ -451,7 +477,7 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
             const float v0 = fmaf(xf, e.y, e.x);
             const int jp = j++;
             const float cp = cm;
-            cm += (float)WIN;
+            next_window();
             if (cls == 0) continue;
             partial = true;
             const cptr<int2> lh = as_cptr(A->lohi) +
@@ -466,12 +492,12 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
                     float val;
                     bool in = (x >= rows.r[m].x) & (x <= rows.r[m].y);
                     if (SENT) {
-                        const float u = v + 0.5f;
+                        const float u = WIDE ? v : v + 0.5f;
                         const float2 pr = lds.pairs[jp * WIN + (int)u];
                         val = fmaf(__builtin_amdgcn_fractf(u), pr.y, pr.x);
                         in = in & !(val <= kEmpty);
                     } else {
-                        const float2 pr = *(const float2*)(pairs + bp_addr(v, cp));
+                        const float2 pr = *(const float2*)(pairs + bp_addr<WIDE>(v, cp));
                         val = fmaf(v, pr.y, pr.x);
                     }
                     acc[k] += in ? val : 0.0f;
@@ -492,7 +518,7 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
             stb(vres, any ? acc[k] * scale : 0.0f, voff, so);
         } else {
             // v = relax * sum / count + v, positivity, sentinel (GBackProj.cu:50-59)
-            float v = fmaf(acc[k], scale, vold[k]);
+            float v = WIDE ? fmaf(relax * acc[k], scale, vold[k]) : fmaf(acc[k], scale, vold[k]);
             const bool empty = !(v > kEmpty);
             v = empty ? kSentinel : (positivity ? fmaxf(v, 0.0f) : v);
             if (any) {
@@ -502,7 +528,8 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
         }
     };
     // every voxel of a wave without partial tiles used the same tilts
-    const float one = (WBP ? 1.0f : relax) * __builtin_amdgcn_rcpf((float)full_cnt);
+    const float num = WBP || WIDE ? 1.0f : relax;
+    const float one = num * __builtin_amdgcn_rcpf((float)full_cnt);
     auto rows = [&](auto all) {
 #pragma unroll
         for (int k = 0; k < TZ; k++) {
@@ -511,7 +538,7 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
                 write(k, one, full_cnt > 0);
             } else {
                 const int count = full_cnt + (int)((cnt[k / 2] >> (k % 2 * 16)) & 0xffffu);
-                write(k, (WBP ? 1.0f : relax) * __builtin_amdgcn_rcpf((float)count), count > 0);
+                write(k, num * __builtin_amdgcn_rcpf((float)count), count > 0);
             }
         }
     };
@@ -521,15 +548,22 @@ __device__ __forceinline__ void bp_tile_body(cptr<BpArgs> A, BpLds<TZ, CH, WBP>&
     if (!WBP && wrote_sent) atomicOr(A->vflag + y, 1);
 }
 
-template <typename S, int TZ, int CH, bool WBP = false>
-__device__ __forceinline__ void bp_tile(cptr<BpArgs> A, BpLds<TZ, CH, WBP>& lds, int xt, int zt,
+template <typename S, int TZ, int CH, int KIND>
+__device__ __forceinline__ void bp_tile(cptr<BpArgs> A, BpLds<TZ, CH, KIND>& lds, int xt, int zt,
                                         int y)
 {
     const cptr<int> sflag = as_cptr(A->sflag);
     if (sflag != nullptr && sflag[y] != 0)
-        bp_tile_body<S, TZ, CH, WBP, true>(A, lds, xt, zt, y);
+        bp_tile_body<S, TZ, CH, KIND, true>(A, lds, xt, zt, y);
     else
-        bp_tile_body<S, TZ, CH, WBP, false>(A, lds, xt, zt, y);
+        bp_tile_body<S, TZ, CH, KIND, false>(A, lds, xt, zt, y);
+}
+
+// SART tiles of a storage type (bp_kind_of on the host).
+template <typename S>
+constexpr int bp_kind()
+{
+    return std::is_same<S, bf16_t>::value ? BP_WIDE : BP_SQUARE;
 }
 
 // n_y > 0: grid (8 x-tiles, z-tiles, slices / 8), n_y slices.  Workgroups go
@@ -539,11 +573,12 @@ __device__ __forceinline__ void bp_tile(cptr<BpArgs> A, BpLds<TZ, CH, WBP>& lds,
 template <typename S, int TZ, int CH>
 __global__ __launch_bounds__(BP_THREADS, 5) void k_back_proj(const BpArgs* __restrict__ a, int n_y)
 {
-    __shared__ BpLds<TZ, CH, false> lds;
+    constexpr int KIND = bp_kind<S>();
+    __shared__ BpLds<TZ, CH, KIND> lds;
     const int per = n_y > 0 ? XCDS : 1;
     const int y = blockIdx.z * per + blockIdx.x % per;
     if (n_y > 0 && y >= n_y) return;
-    bp_tile<S, TZ, CH>(as_cptr(a), lds, blockIdx.x / per, blockIdx.y, y);
+    bp_tile<S, TZ, CH, KIND>(as_cptr(a), lds, blockIdx.x / per, blockIdx.y, y);
 }
 
 // WBP back-projection onto the 2x grid (Recon/GBackProjWbp.cu:14-53): the
@@ -552,11 +587,11 @@ __global__ __launch_bounds__(BP_THREADS, 5) void k_back_proj(const BpArgs* __res
 template <typename S, int TZ>
 __global__ __launch_bounds__(BP_THREADS, 6) void k_wbp_grid_bp(const BpArgs* __restrict__ a, int n_y)
 {
-    __shared__ BpLds<TZ, BP_WBP_CHUNK, true> lds;
+    __shared__ BpLds<TZ, BP_WBP_CHUNK, BP_GRID> lds;
     const int per = n_y > 0 ? XCDS : 1;
     const int y = blockIdx.z * per + blockIdx.x % per;
     if (n_y > 0 && y >= n_y) return;
-    bp_tile<S, TZ, BP_WBP_CHUNK, true>(as_cptr(a), lds, blockIdx.x / per, blockIdx.y, y);
+    bp_tile<S, TZ, BP_WBP_CHUNK, BP_GRID>(as_cptr(a), lds, blockIdx.x / per, blockIdx.y, y);
 }
 
 // Back-projection of many series in persistent launches: blocks take
@@ -569,7 +604,8 @@ __global__ __launch_bounds__(BP_THREADS) void k_back_proj_batch(const BpItem* __
                                                            int total, int* __restrict__ counter)
 {
     constexpr int TZ = (SHAPE & 2) ? 8 : 16, CH = (SHAPE & 1) ? 8 : 16;
-    __shared__ BpLds<TZ, CH, false> lds;
+    constexpr int KIND = bp_kind<S>();
+    __shared__ BpLds<TZ, CH, KIND> lds;
     const cptr<BpItem> E = as_cptr(e);
     int s = 0;
     for (int it = publish_item(claim_item(counter)); it < total;) {
@@ -584,7 +620,7 @@ __global__ __launch_bounds__(BP_THREADS) void k_back_proj_batch(const BpItem* __
             if (r >= nt) break;
             const int zt = r / nx, xt = r - zt * nx;
             if (g > 0) __syncthreads();
-            bp_tile<S, TZ, CH>(&E[s].a, lds, xt, zt, y);
+            bp_tile<S, TZ, CH, KIND>(&E[s].a, lds, xt, zt, y);
         }
         it = publish_item(ahead);
     }
@@ -763,8 +799,9 @@ BpArgs bp_args(const Plan& p, const void* sino, int rows, int first, int n_list,
     a.n_list = n_list;
     a.lohi = p.d_bp_lohi;
     a.lohi_stride = bp_zpad(p.vol_z);
-    a.n_ztiles = bp_ztiles(p.vol_z, p.bp_tz);
-    a.n_xtiles = (p.vol_x + BP_TX - 1) / BP_TX;
+    const int kind = bp_kind_of(p.storage);
+    a.n_ztiles = bp_ztiles(p.vol_z, p.bp_tz, kind);
+    a.n_xtiles = bp_xtiles(p.vol_x, kind);
     a.tiles = p.d_bp_tiles + (size_t)a.n_ztiles * BP_WAVES * a.n_xtiles * first;
     a.relax = relax;
     a.positivity = p.positivity;
@@ -777,9 +814,9 @@ BpArgs bp_args(const Plan& p, const void* sino, int rows, int first, int n_list,
 }
 
 // Grid of a back-projection; *n_y: its argument.
-static dim3 bp_grid(int vol_x, int vol_y, int vol_z, int tz, int* n_y)
+static dim3 bp_grid(int vol_x, int vol_y, int vol_z, int tz, int kind, int* n_y)
 {
-    const int nxt = (vol_x + BP_TX - 1) / BP_TX, nzt = bp_ztiles(vol_z, tz);
+    const int nxt = bp_xtiles(vol_x, kind), nzt = bp_ztiles(vol_z, tz, kind);
     if (vol_y < BP_XCD_SLICES) {
         *n_y = 0;
         return dim3(nxt, nzt, vol_y);
@@ -792,7 +829,7 @@ template <typename S, int TZ, int CH>
 static void launch_bp_v(const Plan& p, int step, hipStream_t s)
 {
     int n_y = 0;
-    const dim3 grid = bp_grid(p.vol_x, p.vol_y, p.vol_z, TZ, &n_y);
+    const dim3 grid = bp_grid(p.vol_x, p.vol_y, p.vol_z, TZ, bp_kind<S>(), &n_y);
     hipLaunchKernelGGL((k_back_proj<S, TZ, CH>), grid, dim3(BP_THREADS), 0, s, p.d_bp_args + step,
                        n_y);
 }
@@ -819,7 +856,7 @@ template <typename S>
 static void launch_wbp_bp_t(const Plan& p, const BpArgs* a, int ny, hipStream_t s)
 {
     int n_y = 0;
-    const dim3 grid = bp_grid(2 * p.vol_x, ny, 2 * p.vol_z, p.bp_tz, &n_y);
+    const dim3 grid = bp_grid(2 * p.vol_x, ny, 2 * p.vol_z, p.bp_tz, BP_GRID, &n_y);
     if (p.bp_tz == 8)
         hipLaunchKernelGGL((k_wbp_grid_bp<S, 8>), grid, dim3(BP_THREADS), 0, s, a, n_y);
     else
