@@ -379,6 +379,9 @@ static atr_status plan_host(Plan& p)
         if (p.fill) fill_table(d.fill_seed, p.aln_x * p.aln_y, h.fill_aln);
         if (p.n_patches > 0)
             h.local.assign(d.local_params, d.local_params + (size_t)p.n * 5 * p.n_patches);
+        if (p.n_patches > 0)
+            p.local_fast = ps_local_fast(d.tilt_axis_deg, d.local_params, p.n, p.n_patches, p.in_x,
+                                         p.in_y, p.aln_x, p.aln_y);
     }
     if (p.binned) {
         FftDesc* fds[4] = {&p.fft_bin_ax, &p.fft_bin_ay, &p.fft_bin_by, &p.fft_bin_bx};
@@ -444,7 +447,7 @@ static atr_status plan_device(Plan& p)
         if ((st = upload(p, &p.d_axis_cs, h.axis_cs, B)) != ATR_OK) return st;
         if ((st = upload(p, &p.d_shifts, h.shifts, B)) != ATR_OK) return st;
         if ((st = dalloc(p, (void**)&p.d_aligned, sizeof(float) * p.n * (size_t)p.aln_x * p.aln_y, B)) != ATR_OK) return st;
-        if ((st = dalloc(p, (void**)&p.d_row_stats, sizeof(double) * 2 * p.n * (size_t)p.aln_y, B)) != ATR_OK) return st;
+        if ((st = dalloc(p, (void**)&p.d_block_stats, sizeof(double) * 2 * p.n * (size_t)ps_blocks(p), B)) != ATR_OK) return st;
         if ((st = dalloc(p, (void**)&p.d_tilt_stats, sizeof(double) * 2 * p.n, B)) != ATR_OK) return st;
         if (p.fill && (st = upload(p, &p.d_fill_aln, h.fill_aln, B)) != ATR_OK) return st;
         if (p.n_patches > 0 && (st = upload(p, &p.d_local, h.local, B)) != ATR_OK) return st;
@@ -539,7 +542,7 @@ static void plan_free(Plan& p)
                      (void**)&p.d_tw_proj, (void**)&p.d_tw_x2, (void**)&p.d_tw_z2,
                      (void**)&p.d_tw_z, (void**)&p.d_tw_x, (void**)&p.d_axis_cs,
                      (void**)&p.d_shifts, (void**)&p.d_excl, (void**)&p.d_aligned,
-                     (void**)&p.d_row_stats, (void**)&p.d_tilt_stats, (void**)&p.d_sino,
+                     (void**)&p.d_block_stats, (void**)&p.d_tilt_stats, (void**)&p.d_sino,
                      (void**)&p.d_diff, (void**)&p.d_vol, (void**)&p.d_sflag, (void**)&p.d_vflag,
                      (void**)&p.d_vstats, (void**)&p.d_wbp_t, (void**)&p.d_wbp_u,
                      (void**)&p.d_bp_args, (void**)&p.d_fp_args, (void**)&p.d_wbp_grid,

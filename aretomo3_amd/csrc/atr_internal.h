@@ -64,6 +64,9 @@ inline int bp_default_tz(int vol_x, int vol_y, int vol_z, int kind)
     const long tiles = (long)bp_xtiles(vol_x, kind) * bp_ztiles(vol_z, 16, kind) * vol_y;
     return tiles < 1024 ? 8 : 16;
 }
+// Pre-stage: aligned rows per workgroup (with patches, three FP64 sums per row
+// are held in registers).
+constexpr int ps_rows(bool local) { return local ? 16 : 32; }
 // Forward projection: a workgroup of FP_THREADS owns one slice and a group of
 // tilts; wave w takes the (tilt, 64-ray tile) pairs w, w+16, ... (FP_MAXP at
 // most), so every wave sees every tilt; the slice is streamed through LDS in
@@ -236,7 +239,8 @@ struct Plan {
     float2* d_bin_u = nullptr;        // [N][bin_y][bin_x/2+1] cropped, column-inverted
     float2* d_tw_bin[4] = {nullptr, nullptr, nullptr, nullptr};
     FftDesc fft_bin_ax{}, fft_bin_ay{}, fft_bin_by{}, fft_bin_bx{};
-    double* d_row_stats = nullptr;    // [N][aln_y][2] per-row (sum, count) of non-empty pixels
+    double* d_block_stats = nullptr;  // [N][ps_blocks][2] (sum, count) of non-empty pixels
+    bool local_fast = false;          // patch weights as products (ps_local_fast)
     double* d_tilt_stats = nullptr;   // [N][2] (sum, count) of non-empty aligned pixels
     void* d_sino = nullptr;           // [vol_y][N][sino_stride] weighted projections
     void* d_diff = nullptr;           // [vol_y][max_subset][sino_stride]
@@ -462,6 +466,8 @@ void fp_pair_schedule(const Geometry& g, const int* list, int n_list, int proj, 
                       std::vector<int>& tab, int n_waves = FP_WAVES);
 void split_items(int n_items, int n_splits, std::vector<int>& starts, std::vector<int>& sizes);
 void fill_table(uint64_t seed, int n, std::vector<int>& table);
+bool ps_local_fast(const float* axis_deg, const float* local, int n, int n_patches, int in_x, int in_y,
+                   int aln_x, int aln_y);
 void aligned_size(int raw_x, int raw_y, float axis_deg, int* ax, int* ay);
 bool make_fft(int n, FftDesc& fd);
 std::vector<float2> twiddles(int n);
@@ -470,6 +476,7 @@ uint64_t splitmix64(uint64_t x);
 
 // ---- kernel launchers (kernels_*.hip) -----------------------------------
 void launch_prestage(const Plan& p, const float* in, hipStream_t s);
+int ps_blocks(const Plan& p);   // pre-stage workgroups per tilt
 void launch_tilt_stats(const Plan& p, hipStream_t s);
 void launch_bin(const Plan& p, const float* in, hipStream_t s);
 // Volume dimensions a plan for *d would produce (validates the descriptor).

@@ -72,6 +72,34 @@ void aligned_size(int raw_x, int raw_y, float axis_deg, int* ax, int* ay)
     *ay = raw_x;
 }
 
+// Whether the pre-stage may form the patch weights of every tilt as products
+// exp(a_p x + c_p) exp(b_p y): all exponents within +-300, so that neither
+// factor nor product leaves the range of a double, and the weights as written,
+// exp(-100 d^2), above e^-600, so that none of them is 0.
+bool ps_local_fast(const float* axis_deg, const float* local, int n, int n_patches, int in_x, int in_y,
+                   int aln_x, int aln_y)
+{
+    for (int t = 0; t < n; t++) {
+        const float ang = axis_deg[t] * (3.141592654f / 180.0f);
+        const double ca = std::cos((double)ang), sa = std::sin((double)ang);
+        const double hx = aln_x * 0.5, hy = aln_y * 0.5;
+        const double rx = (std::fabs(hx * ca) + std::fabs(hy * sa)) / in_x;
+        const double ry = (std::fabs(hx * sa) + std::fabs(hy * ca)) / in_y;
+        const double quad = 100.0 * (rx * rx + ry * ry);
+        const float* lp = local + (size_t)t * 5 * n_patches;
+        for (int q = 0; q < n_patches; q++) {
+            if (lp[4 * n_patches + q] < 0.9f) continue;
+            const double cx = lp[q], cy = lp[n_patches + q];
+            const double gx = 200.0 * cx / ((double)in_x * in_x);
+            const double gy = 200.0 * cy / ((double)in_y * in_y);
+            const double e = std::fabs(gx * ca + gy * sa) * hx + std::fabs(gy * ca - gx * sa) * hy +
+                             0.5 * (gx * cx + gy * cy);
+            if (!(e <= 300.0) || !(quad + e <= 600.0)) return false;
+        }
+    }
+    return true;
+}
+
 // Interval {lo, hi} of integer i in [0, n) where pred(i) holds, for a
 // predicate that holds on one contiguous run (monotone geometry).  Empty
 // interval = {n, -1}.
@@ -151,53 +179,70 @@ void build_bp_tiles(const std::vector<BpTilt>& lists, const std::vector<int>& en
     const size_t per = (size_t)nzt * nxt * BP_WAVES;
     const int total = ends.back(), stride = bp_zpad(vol_z);
     tiles.assign(per * total + BP_PAD, int2{0, 0});
-    parallel_tilts(total, [&](int l) {
-        int first = 0, seg = 0;
-        while (ends[seg] <= l) first = ends[seg++];
-        const int len = ends[seg] - first, t = lists[l].tilt;
-        int2* out = tiles.data() + per * first + (l - first);
-        const double c = cs[2 * t], s = cs[2 * t + 1];
-        const int2* lh = lohi.data() + (size_t)t * stride;
-        for (int zt = 0; zt < nzt; zt++) {
-            // per row of waves: the intervals' overlap and union over its rows
-            int in_lo[BP_WAVES], in_hi[BP_WAVES], any_lo[BP_WAVES], any_hi[BP_WAVES];
+    // One row of tiles of every list: per tilt the rows of waves' intervals
+    // (their overlap and union) first, then the entries in the order they lie.
+    struct Row {
+        int in_lo[BP_WAVES], in_hi[BP_WAVES], any_lo[BP_WAVES], any_hi[BP_WAVES];
+        double c, s, sz;
+    };
+    auto build = [&](int zt) {
+        const int zt0 = zt * wz * tz;
+        const double fz0 = zt0 - vol_z * 0.5, fz1 = fz0 + (wz * tz - 1);
+        std::vector<Row> rows(total);
+        for (int l = 0; l < total; l++) {
+            Row& r = rows[l];
+            const int t = lists[l].tilt;
+            const int2* lh = lohi.data() + (size_t)t * stride;
+            r.c = cs[2 * t], r.s = cs[2 * t + 1];
+            r.sz = std::min(r.s * fz0, r.s * fz1);
             for (int w = 0; w < wz; w++) {
-                const int z0 = (zt * wz + w) * tz, z1 = std::min(z0 + tz, vol_z);
-                in_lo[w] = 0, in_hi[w] = z0 < vol_z ? vol_x : -1;
-                any_lo[w] = vol_x, any_hi[w] = -1;
+                const int z0 = zt0 + w * tz, z1 = std::min(z0 + tz, vol_z);
+                r.in_lo[w] = 0, r.in_hi[w] = z0 < vol_z ? vol_x : -1;
+                r.any_lo[w] = vol_x, r.any_hi[w] = -1;
                 for (int z = z0; z < z1; z++) {
-                    in_lo[w] = std::max(in_lo[w], lh[z].x);
-                    in_hi[w] = std::min(in_hi[w], lh[z].y);
+                    r.in_lo[w] = std::max(r.in_lo[w], lh[z].x);
+                    r.in_hi[w] = std::min(r.in_hi[w], lh[z].y);
                     if (lh[z].y >= lh[z].x) {
-                        any_lo[w] = std::min(any_lo[w], lh[z].x);
-                        any_hi[w] = std::max(any_hi[w], lh[z].y);
+                        r.any_lo[w] = std::min(r.any_lo[w], lh[z].x);
+                        r.any_hi[w] = std::max(r.any_hi[w], lh[z].y);
                     }
                 }
             }
-            const int zt0 = zt * wz * tz;
-            const double fz0 = zt0 - vol_z * 0.5, fz1 = fz0 + (wz * tz - 1);
-            const double sz = std::min(s * fz0, s * fz1);
+        }
+        int first = 0;
+        for (int end : ends) {
+            const int len = end - first;
+            int2* out = tiles.data() + per * first;
             for (int xt = 0; xt < nxt; xt++) {
                 const int x0 = xt * wx * BP_TX, x1 = std::min(x0 + wx * BP_TX, vol_x) - 1;
                 const double fx0 = x0 - vol_x * 0.5, fx1 = x1 - vol_x * 0.5;
-                const int w0 = (int)std::floor(offset + scale * (std::min(c * fx0, c * fx1) + sz)) - 3;
                 for (int w = 0; w < BP_WAVES; w++) {
                     const int xw = w % wx, zw = w / wx;
                     const int xa = x0 + xw * BP_TX, xb = std::min(xa + BP_TX, vol_x) - 1;
-                    const int z0 = zt0 + zw * tz;
-                    // (columns between the rows' intervals count as partial)
-                    const bool full = xa <= xb && in_lo[zw] <= xa && in_hi[zw] >= xb;
-                    const bool any = xa <= xb && any_lo[zw] <= xb && any_hi[zw] >= xa;
-                    const float u00 =
-                        kind == BP_WIDE
-                            ? (float)(scale * (c * fx0 + s * fz0) + offset - w0)
-                            : (float)(scale * (c * fx0 + s * (z0 - vol_z * 0.5)) + offset - w0 - 0.5);
-                    out[((size_t)(zt * wz + zw) * (nxt * wx) + xt * wx + xw) * len] =
-                        int2{4 * w0 + (full ? 1 : (any ? 2 : 0)), __builtin_bit_cast(int, u00)};
+                    const double fzw = zt0 + zw * tz - vol_z * 0.5;
+                    int2* o = out + ((size_t)(zt * wz + zw) * (nxt * wx) + xt * wx + xw) * len;
+                    for (int l = 0; l < len; l++) {
+                        const Row& r = rows[first + l];
+                        const double c = r.c, s = r.s;
+                        const int w0 =
+                            (int)std::floor(offset + scale * (std::min(c * fx0, c * fx1) + r.sz)) - 3;
+                        // (columns between the rows' intervals count as partial)
+                        const bool full = xa <= xb && r.in_lo[zw] <= xa && r.in_hi[zw] >= xb;
+                        const bool any = xa <= xb && r.any_lo[zw] <= xb && r.any_hi[zw] >= xa;
+                        const float u00 =
+                            kind == BP_WIDE ? (float)(scale * (c * fx0 + s * fz0) + offset - w0)
+                                            : (float)(scale * (c * fx0 + s * fzw) + offset - w0 - 0.5);
+                        o[l] = int2{4 * w0 + (full ? 1 : (any ? 2 : 0)), __builtin_bit_cast(int, u00)};
+                    }
                 }
             }
+            first = end;
         }
-    });
+    };
+    // host threads pay from a few milliseconds of work on
+    if (per * total > (1u << 16)) parallel_for(nzt, build);
+    else
+        for (int zt = 0; zt < nzt; zt++) build(zt);
 }
 
 std::vector<BpTilt> bp_list(const std::vector<float>& cs, const std::vector<TiltRow>& rows, float scale)
