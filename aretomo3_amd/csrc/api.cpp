@@ -17,6 +17,7 @@
 #include <tuple>
 
 #include "atr_internal.h"
+#include "fft_reg.h"
 
 namespace atr {
 
@@ -143,6 +144,7 @@ static atr_status plan_sizes(const atr_series_desc* d, Plan& p)
                         "Fourier binning: image size has no FFT plan");
         if (p.aln_x > 8192 || p.aln_y > 8192)
             return fail(ATR_ERR_UNSUPPORTED_SIZE, "Fourier binning supports images up to 8192");
+        p.bin_kb = fft_col_width(p.aln_y, p.bin_y);
     }
     p.fill = p.prestage && (d->random_fill != 0 || p.binned);
     // CDoWbpRecon.cpp:37-38, GBackProj.cu:74: VolX = ProjX/2*2 = effective ProjX
@@ -213,6 +215,7 @@ static atr_status plan_sizes(const atr_series_desc* d, Plan& p)
             return fail(ATR_ERR_UNSUPPORTED_SIZE,
                         "WBP supports ProjX (= VolX) <= 2048 and VolZ <= 2048");
         // slab of slices whose spectra are buffered between the WBP kernels
+        p.wbp_kb = fft_col_width(2 * p.vol_z, p.vol_z);
         size_t per_slice = (size_t)3 * p.vol_z * (p.vol_x / 2 + 1) * sizeof(float2) +
                            (size_t)4 * p.vol_z * p.vol_x * sizeof(float);
         size_t budget = (size_t)1 << 30;
@@ -231,8 +234,8 @@ static size_t plan_bytes_estimate(const Plan& p)
         b += n * 5 * (size_t)p.n_patches * 4;
     }
     if (p.binned) {
-        size_t kx = p.bin_x / 2 + 1;
-        b += n * (size_t)p.bin_x * p.bin_y * 4 + n * kx * (p.aln_y + p.bin_y) * 8;
+        const int kx = p.bin_x / 2 + 1;
+        b += n * (size_t)p.bin_x * p.bin_y * 4 + n * spec_elems(kx, p.aln_y + p.bin_y, p.bin_kb) * 8;
         b += (size_t)(p.aln_x + p.aln_y + p.bin_x + p.bin_y) * 8;
     }
     b += (size_t)p.vol_y * n * p.sino_stride * sb;
@@ -245,7 +248,7 @@ static size_t plan_bytes_estimate(const Plan& p)
         const int kind = bp_kind_of(p.storage);
         b += 2 * n * (size_t)bp_ztiles(p.vol_z, 8, kind) * bp_xtiles(p.vol_x, kind) * BP_WAVES * sizeof(int2);
     } else {
-        b += (size_t)p.wbp_slab * 3 * p.vol_z * (p.vol_x / 2 + 1) * sizeof(float2);
+        b += p.wbp_slab * spec_elems(p.vol_x / 2 + 1, 3 * p.vol_z, p.wbp_kb) * sizeof(float2);
         b += (size_t)p.wbp_slab * 4 * p.vol_z * p.vol_x * sizeof(float);
         b += n * 2 * p.vol_z * 8 + n * 16;
         b += n * (size_t)bp_ztiles(2 * p.vol_z, 8, BP_GRID) * bp_xtiles(2 * p.vol_x, BP_GRID) * BP_WAVES * sizeof(int2);
@@ -455,8 +458,8 @@ static atr_status plan_device(Plan& p)
     if (p.binned) {
         const int kx = p.bin_x / 2 + 1;
         if ((st = dalloc(p, (void**)&p.d_binned, sizeof(float) * p.n * (size_t)p.bin_x * p.bin_y, B)) != ATR_OK) return st;
-        if ((st = dalloc(p, (void**)&p.d_bin_t, sizeof(float2) * p.n * (size_t)kx * p.aln_y, B)) != ATR_OK) return st;
-        if ((st = dalloc(p, (void**)&p.d_bin_u, sizeof(float2) * p.n * (size_t)kx * p.bin_y, B)) != ATR_OK) return st;
+        if ((st = dalloc(p, (void**)&p.d_bin_t, sizeof(float2) * p.n * spec_elems(kx, p.aln_y, p.bin_kb), B)) != ATR_OK) return st;
+        if ((st = dalloc(p, (void**)&p.d_bin_u, sizeof(float2) * p.n * spec_elems(kx, p.bin_y, p.bin_kb), B)) != ATR_OK) return st;
         FftDesc* fds[4] = {&p.fft_bin_ax, &p.fft_bin_ay, &p.fft_bin_by, &p.fft_bin_bx};
         for (int i = 0; i < 4; i++) {
             if ((st = upload(p, &p.d_tw_bin[i], h.tw_bin[i], B)) != ATR_OK) return st;
@@ -521,9 +524,9 @@ static atr_status plan_device(Plan& p)
         p.fft_z2.tw = p.d_tw_z2;
         p.fft_z.tw = p.d_tw_z;
         p.fft_x.tw = p.d_tw_x;
-        size_t kxn = p.vol_x / 2 + 1;
-        if ((st = dalloc(p, (void**)&p.d_wbp_t, (size_t)p.wbp_slab * 2 * p.vol_z * kxn * sizeof(float2), B)) != ATR_OK) return st;
-        if ((st = dalloc(p, (void**)&p.d_wbp_u, (size_t)p.wbp_slab * p.vol_z * kxn * sizeof(float2), B)) != ATR_OK) return st;
+        const int kxn = p.vol_x / 2 + 1;
+        if ((st = dalloc(p, (void**)&p.d_wbp_t, p.wbp_slab * spec_elems(kxn, 2 * p.vol_z, p.wbp_kb) * sizeof(float2), B)) != ATR_OK) return st;
+        if ((st = dalloc(p, (void**)&p.d_wbp_u, p.wbp_slab * spec_elems(kxn, p.vol_z, p.wbp_kb) * sizeof(float2), B)) != ATR_OK) return st;
     }
     // a stream-ordered upload still reads the host tables: the caller drops
     // them once the stream has passed (plan_drop_host_tables)

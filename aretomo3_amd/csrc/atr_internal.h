@@ -235,8 +235,8 @@ struct Plan {
     float* d_aligned = nullptr;       // [N][aln_y][aln_x] pre-stage output with sentinels
     float* d_local = nullptr;         // [N][5][n_patches] patch centres, shifts, good flags
     float* d_binned = nullptr;        // [N][bin_y][bin_x] Fourier-binned images
-    float2* d_bin_t = nullptr;        // [N][aln_y][bin_x/2+1] row spectra
-    float2* d_bin_u = nullptr;        // [N][bin_y][bin_x/2+1] cropped, column-inverted
+    float2* d_bin_t = nullptr;        // [N][blocks][aln_y][bin_kb] row spectra
+    float2* d_bin_u = nullptr;        // [N][blocks][bin_y][bin_kb] cropped, column-inverted
     float2* d_tw_bin[4] = {nullptr, nullptr, nullptr, nullptr};
     FftDesc fft_bin_ax{}, fft_bin_ay{}, fft_bin_by{}, fft_bin_bx{};
     double* d_block_stats = nullptr;  // [N][ps_blocks][2] (sum, count) of non-empty pixels
@@ -258,9 +258,10 @@ struct Plan {
     FpArgs* d_fp_args = nullptr;      // per subset
     float* d_wbp_grid = nullptr;      // [slab][2VolZ][2VolX] the 2x-grid back-projection
     int2* d_wbp_tiles = nullptr;      // the 2x grid's, as bp_tiles
-    float2* d_wbp_t = nullptr;        // [slab][2VolZ][VolX/2+1]
-    float2* d_wbp_u = nullptr;        // [slab][VolZ][VolX/2+1]
+    float2* d_wbp_t = nullptr;        // [slab][blocks][2VolZ][wbp_kb]
+    float2* d_wbp_u = nullptr;        // [slab][blocks][VolZ][wbp_kb]
     int wbp_slab = 0;
+    int wbp_kb = 8, bin_kb = 8;       // columns per block of the spectra
     size_t device_bytes = 0;
     // FFT descriptors
     FftDesc fft_proj{}, fft_x2{}, fft_z2{}, fft_z{}, fft_x{};
@@ -481,12 +482,12 @@ void launch_tilt_stats(const Plan& p, hipStream_t s);
 void launch_bin(const Plan& p, const float* in, hipStream_t s);
 // Volume dimensions a plan for *d would produce (validates the descriptor).
 atr_status desc_volume(const atr_series_desc* d, int* vol_x, int* vol_y, int* vol_z);
-int bin_col_block(int ay);
 void launch_weight_sart(const Plan& p, const float* in, hipStream_t s);
 void launch_filter_wbp(const Plan& p, const float* in, hipStream_t s);
 void launch_zero(float* ptr, size_t n, hipStream_t s);
 void launch_zero_int(int* ptr, int n, hipStream_t s);
-int wbp_col_block(int vol_z);
+// entries of one slice's half spectrum in blocks of kb columns
+size_t spec_elems(int columns, int rows, int kb);
 // first: offset of the list in p.d_lists
 BpArgs bp_args(const Plan& p, const void* sino, int rows, int first, int n_list, float relax,
                bool check_sent);

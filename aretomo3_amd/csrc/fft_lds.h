@@ -22,9 +22,11 @@ struct FftDesc {
     const float2* tw;  // n entries
 };
 
+// The fused form is written out: left to the compiler, which of the products is
+// rounded first depends on the kernel around it.
 __device__ __forceinline__ float2 cmul(float2 a, float2 b)
 {
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+    return make_float2(__builtin_fmaf(a.x, b.x, -(a.y * b.y)), __builtin_fmaf(a.y, b.x, a.x * b.y));
 }
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
@@ -73,6 +75,11 @@ __device__ __forceinline__ void dft_small(float2* v, float sign)
     }
 }
 
+// x / d for 0 <= x < 2^21, d <= 8192, inv = 1 / d rounded: three instructions in
+// place of an integer division (the sum is at least 0.5 / d from an integer,
+// the rounding errors are below x / d 2^-22).
+__device__ __forceinline__ int fft_div(int x, float inv) { return (int)(((float)x + 0.5f) * inv); }
+
 template <int R>
 __device__ __forceinline__ void fft_stage(const float2* __restrict__ src, float2* __restrict__ dst,
                                           int n, int batch, int ns, const float2* __restrict__ tw,
@@ -81,12 +88,13 @@ __device__ __forceinline__ void fft_stage(const float2* __restrict__ src, float2
     const int m = n / R;          // butterflies per sequence
     const int step = n / (ns * R);
     const int total = batch * m;
+    const float inv_m = 1.0f / (float)m, inv_ns = 1.0f / (float)ns;
     for (int idx = tid; idx < total; idx += nthreads) {
-        int bi = idx / m;
+        int bi = fft_div(idx, inv_m);
         int j = idx - bi * m;
         const float2* s = src + bi * n;
         float2* d = dst + bi * n;
-        int k = j % ns;
+        int jn = fft_div(j, inv_ns), k = j - jn * ns;
         float2 v[R];
 #pragma unroll
         for (int r = 0; r < R; r++) v[r] = s[j + r * m];
@@ -99,7 +107,7 @@ __device__ __forceinline__ void fft_stage(const float2* __restrict__ src, float2
             }
         }
         dft_small<R>(v, sign);
-        int o = (j / ns) * ns * R + k;
+        int o = jn * ns * R + k;
 #pragma unroll
         for (int r = 0; r < R; r++) d[o + r * ns] = v[r];
     }
@@ -117,13 +125,13 @@ __device__ __forceinline__ void fft_stage_any(const float2* __restrict__ src, fl
     const int m = n / R;
     const int step = n / (ns * R);
     const int total = batch * n;
+    const float inv_n = 1.0f / (float)n, inv_ns = 1.0f / (float)ns, inv_r = 1.0f / (float)R;
     for (int idx = tid; idx < total; idx += nthreads) {
-        int bi = idx / n;
+        int bi = fft_div(idx, inv_n);
         int pos = idx - bi * n;
-        int k = pos % ns;
-        int t = pos / ns;
-        int q = t % R;
-        int j = (t / R) * ns + k;
+        int t = fft_div(pos, inv_ns), k = pos - t * ns;
+        int tr = fft_div(t, inv_r), q = t - tr * R;
+        int j = tr * ns + k;
         const float2* s = src + bi * n;
         int c = k * step + q * m;
         int e = 0;
