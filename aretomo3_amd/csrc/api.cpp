@@ -244,6 +244,8 @@ static size_t plan_bytes_estimate(const Plan& p)
         b += vox * 4 + (size_t)p.vol_y * p.max_subset * p.sino_stride * sb;
         b += n * p.vol_z * 8 + n * p.proj * 8 + (size_t)p.vol_x * p.vol_z * 4;
         b += n * (size_t)(p.vol_z * 2.5 + 16) * 16;  // FP sample tables (bounded by 60 deg)
+        const int bz = fp_balanced_rows(fp_band_rows(p.vol_x), p.vol_z);
+        b += fp_part_bytes(p, (p.vol_z - 1 + bz - 1) / bz, bz);
         // back-projection tiles: every tilt is in the initial list and in a subset's
         const int kind = bp_kind_of(p.storage);
         b += 2 * n * (size_t)bp_ztiles(p.vol_z, 8, kind) * bp_xtiles(p.vol_x, kind) * BP_WAVES * sizeof(int2);
@@ -321,6 +323,17 @@ static atr_status sart_tables_device(Plan& p)
     if ((st = reupload(p, &p.d_fp_geo, g.fp_geo, B, p.tab_bytes[4])) != ATR_OK) return st;
     if ((st = reupload(p, &p.d_fp_desc, g.fp_desc, B, p.tab_bytes[5])) != ATR_OK) return st;
     if ((st = reupload(p, &p.d_fp_pairs, p.host.sched, B, p.tab_bytes[6])) != ATR_OK) return st;
+    const size_t part = fp_part_bytes(p, g.fp_nbands, g.fp_bz);
+    if (part != p.fp_part_alloc) {
+        if (p.d_fp_part) {
+            plan_mfree(p, p.d_fp_part);
+            p.d_fp_part = nullptr;
+            B -= p.fp_part_alloc;
+        }
+        p.fp_part_alloc = 0;
+        if (part && (st = dalloc(p, (void**)&p.d_fp_part, part, B)) != ATR_OK) return st;
+        p.fp_part_alloc = part;
+    }
     // kernel arguments of every SART step, read by the kernels from device
     // memory: [0] initial back-projection, [1 + s] subset s
     const int n_all = (int)p.all_tilts.size();
@@ -548,7 +561,7 @@ static void plan_free(Plan& p)
                      (void**)&p.d_block_stats, (void**)&p.d_tilt_stats, (void**)&p.d_sino,
                      (void**)&p.d_diff, (void**)&p.d_vol, (void**)&p.d_sflag, (void**)&p.d_vflag,
                      (void**)&p.d_vstats, (void**)&p.d_wbp_t, (void**)&p.d_wbp_u,
-                     (void**)&p.d_bp_args, (void**)&p.d_fp_args, (void**)&p.d_wbp_grid,
+                     (void**)&p.d_bp_args, (void**)&p.d_fp_args, (void**)&p.d_fp_part, (void**)&p.d_wbp_grid,
                      (void**)&p.d_wbp_tiles, (void**)&p.d_local, (void**)&p.d_binned,
                      (void**)&p.d_bin_t, (void**)&p.d_bin_u, (void**)&p.d_tw_bin[0],
                      (void**)&p.d_tw_bin[1], (void**)&p.d_tw_bin[2], (void**)&p.d_tw_bin[3]};
@@ -557,6 +570,7 @@ static void plan_free(Plan& p)
         *q = nullptr;
     }
     for (size_t& b : p.tab_bytes) b = 0;
+    p.fp_part_alloc = 0;
     p.device_bytes = 0;
     for (auto& e : p.ev_pool) (void)hipEventDestroy(e);
     for (auto& e : p.ev_pending) {

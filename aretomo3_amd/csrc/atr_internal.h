@@ -79,6 +79,18 @@ constexpr int FP_LDS_BUDGET = 150 * 1024;
 constexpr int FP_BZ_MAX = 17;                // cell rows per band at most
 constexpr int FP_STAGE_ROWS = 9;              // rows a thread loads before forming pairs
 constexpr int FP_RP_ISSUE = 8;                // register prefetch: pair slots before its loads
+// Few (slice, tilt group) items: up to this many, the bands of a slice are
+// projected side by side (k_fp_part, k_fp_sum).  Measured per pass (4
+// iterations, 5 subsets of 41 tilts), bands in turn / side by side:
+// 1024 x 8 x 256 (items 8) 4.05 / 0.68 ms, 1024 x 128 5.67 / 4.95, 1024 x 256
+// 6.97 / 9.77; 700 x 100 x 300 4.93 / 3.48, 700 x 200 5.84 / 6.55.  Where two
+// workgroups' bands fit the LDS of a CU the line lies higher: 512 x 256 x 128
+// 2.41 / 2.19, 300 x 300 x 100 2.41 / 1.77.
+constexpr int FP_SPLIT_ITEMS = 128, FP_SPLIT_ITEMS_TWO = 384;
+constexpr int FP_LDS_TWO = 80 * 1024;         // bands of which two fit the LDS
+constexpr size_t FP_SPLIT_BYTES = 256 << 20;  // the bands' sums at most
+// workgroups up to which a band's pair slots are shared out, and shares
+constexpr int FP_SPLIT_GROUPS = 256, FP_SPLIT_SHARES = 4;
 // Band-prefetching variant: the last wave streams the next band's volume rows
 // into LDS with direct global->LDS loads while the other waves sample the
 // current band; the raw rows sit after the pair rows.  Needs VolX % 256 == 0
@@ -256,6 +268,9 @@ struct Plan {
     size_t tab_bytes[9] = {0};        // sizes of the tile-shape dependent tables
     BpArgs* d_bp_args = nullptr;      // SART step arguments: initial BP, then per subset
     FpArgs* d_fp_args = nullptr;      // per subset
+    float* d_fp_part = nullptr;       // FpArgs::part; null: fp_block does it
+    size_t fp_part_alloc = 0;
+    bool queued = false;              // only run in work-queue launches (serve)
     float* d_wbp_grid = nullptr;      // [slab][2VolZ][2VolX] the 2x-grid back-projection
     int2* d_wbp_tiles = nullptr;      // the 2x grid's, as bp_tiles
     float2* d_wbp_t = nullptr;        // [slab][blocks][2VolZ][wbp_kb]
@@ -310,6 +325,7 @@ struct FpArgs {
     void* diff;
     int diff_rows;
     int pf;                    // band-prefetching variant (fp_waves(pf) sampling waves)
+    float* part;               // few slices: [bands][vol_y][diff_rows][stride] sums, then counts
 };
 // Entries of the batched (work-queue) launches; item0 = first queue index.
 // shape: the series' back-projection tile shape, bp_shape(bp_tz, bp_chunk).
@@ -491,6 +507,7 @@ size_t spec_elems(int columns, int rows, int kb);
 // first: offset of the list in p.d_lists
 BpArgs bp_args(const Plan& p, const void* sino, int rows, int first, int n_list, float relax,
                bool check_sent);
+size_t fp_part_bytes(const Plan& p, int n_bands, int bz);
 FpArgs fp_args(const Plan& p, const int* fp_list, int n_list, const int* sched);
 size_t fp_lds_bytes(int bz, int vol_x, int pf = 0);
 // step 0: initial back-projection, 1 + s: subset s (arguments in p.d_bp_args)

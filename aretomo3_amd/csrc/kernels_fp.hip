@@ -142,6 +142,19 @@ __device__ __forceinline__ void fp_run(const char* __restrict__ band, int rowb_r
     }
 }
 
+// A ray's sum of `count` samples to the difference raw - forward projection.
+template <typename S>
+__device__ __forceinline__ void fp_store_diff(cptr<FpArgs> A, int y, int j, int t, int xd, float sum,
+                                              int count)
+{
+    const int stride = A->stride;
+    const float fwd = count <= 0 ? kSentinel : sum / (float)count;
+    float raw = ldg((gptr<const S>)A->sino + ((size_t)y * A->n + t) * stride + xd);
+    if (raw <= empty_threshold<S>()) raw = kSentinel;
+    const float d = (fwd < kEmpty || raw < kEmpty) ? 0.0f : raw - fwd;
+    stg((gptr<S>)A->diff + ((size_t)y * A->diff_rows + j) * stride + xd, d);
+}
+
 // One (group of tilts, slice) work item.  Returns early, for the whole
 // block, when the slice's sentinel flag does not match SENT.  Ends after a
 // barrier, with the LDS free for the next item.
@@ -186,10 +199,6 @@ __device__ __forceinline__ void fp_block(cptr<FpArgs> A, float2* __restrict__ ba
     const cptr<float4> geo = as_cptr(A->geo);
     const cptr<int4> fp_desc = as_cptr(A->fp_desc);
     const int nb = A->nb, bz = A->bz, proj = A->proj;
-    const gptr<const S> sino = (gptr<const S>)A->sino;
-    const int n = A->n, stride = A->stride;
-    const gptr<S> diff = (gptr<S>)A->diff;
-    const int diff_rows = A->diff_rows;
     if ((as_cptr(A->vflag)[y] != 0) != SENT) return;
     const int tid = threadIdx.x, lane = tid & 63;
     // wave index made provably uniform so that all per-pair table reads are
@@ -426,11 +435,7 @@ __device__ __forceinline__ void fp_block(cptr<FpArgs> A, float2* __restrict__ ba
             const int xd = ((jt & 0xffffff) - t * ntile) * FP_WAVE + lane;
             if (xd < proj) {
                 const int count = SENT ? cnt[i] : fp_range[(size_t)t * proj + xd].y;
-                const float fwd = count <= 0 ? kSentinel : acc[i] / (float)count;
-                float raw = ldg(sino + ((size_t)y * n + t) * stride + xd);
-                if (raw <= empty_threshold<S>()) raw = kSentinel;
-                const float d = (fwd < kEmpty || raw < kEmpty) ? 0.0f : raw - fwd;
-                stg(diff + ((size_t)y * diff_rows + j) * stride + xd, d);
+                fp_store_diff<S>(A, y, j, t, xd, acc[i], count);
             }
         }
     }
@@ -449,6 +454,114 @@ __global__ __launch_bounds__(FP_THREADS) void k_for_proj_diff(const FpArgs* __re
     // before it left in the 256 MB memory-side cache (1024^2 x 256: 1.140 ->
     // 1.115 ms here, 0.569 -> 0.550 ms in the back-projection)
     fp_block<S, SENT, ROWB, PF, RP>(as_cptr(a), band, blockIdx.x, gridDim.y - 1 - blockIdx.y);
+}
+
+// ------------------------------------------------------------------------
+// The same for few slices, in two launches: k_fp_part has a workgroup per
+// (slice, group of tilts, band, share of the pair slots) and stores the sum of
+// each ray's samples in its band, k_fp_sum adds a ray's bands in the order in
+// which fp_block does and writes the difference, so the results are the same
+// bits.  Slices with and without empty voxels go through one launch.
+//
+// fp_block walks the bands of a slice one after the other: with one slice of
+// 512 x 128 that is one busy CU, and 65 us for 8 tilts of 512 rays, of which
+// the samples are 4; with the bands side by side the two launches take FPP_US.
+// ------------------------------------------------------------------------
+template <bool SENT>
+__device__ __forceinline__ void fp_part_band(cptr<FpArgs> A, float2* __restrict__ band, int gx, int y,
+                                             int vol_y, int b, int slot0, int slot_step)
+{
+    const int vol_x = A->vol_x, vol_z = A->vol_z, nb = A->nb, bz = A->bz, proj = A->proj;
+    const cptr<int> fp_list = as_cptr(A->fp_list);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j0 = gx * A->group;
+    const int ntile = (proj + FP_WAVE - 1) / FP_WAVE;
+    const cptr<int> pair_tab = as_cptr(A->sched) + (size_t)gx * (FP_WAVES * FP_MAXP) + wave * FP_MAXP;
+    const int pitch = vol_x + 1, rowb = pitch * (int)sizeof(float2);
+    const float xmax1 = (float)(vol_x - 1);
+    const int zb = b * bz, rows = min(bz, vol_z - 1 - zb) + 1;
+    const gptr<const float> V = as_gptr(A->vol) + ((size_t)y * vol_z + zb) * vol_x;
+    // a wave per row, so that all loads of the band are in flight at once
+    for (int r = wave; r < rows; r += FP_WAVES) {
+#pragma unroll 4
+        for (int col = lane; col < pitch; col += 64) {
+            const int xi = col - 1, xa = max(xi, 0), xb = min(xa + 1, vol_x - 1);
+            const float va = V[r * vol_x + xa], vb = V[r * vol_x + xb];
+            const float dx = vb - va;
+            const float v0 = SENT ? (xi < 0 ? va - dx : va) : fmaf(-(float)max(col, 1), dx, va);
+            band[r * pitch + col] = make_float2(v0, dx);
+        }
+    }
+    __syncthreads();
+    const gptr<float> part = as_gptr(A->part) + ((size_t)b * vol_y + y) * A->diff_rows * A->stride;
+    const gptr<uint16_t> part_n =
+        (gptr<uint16_t>)(as_gptr(A->part) + (size_t)nb * vol_y * A->diff_rows * A->stride) +
+        ((size_t)b * vol_y + y) * A->diff_rows * A->stride;
+    for (int i = slot0; i < FP_MAXP; i += slot_step) {
+        const int jt = pair_tab[i];
+        if (jt < 0) continue;
+        const int j = j0 + (jt >> 24), t = fp_list[j], tile = (jt & 0xffffff) - t * ntile;
+        const int xd = tile * FP_WAVE + lane;
+        const int4 d = ldc(as_cptr(A->fp_desc) + (size_t)(jt & 0xffffff) * nb + b);
+        const float tf1 = (float)(((double)min(xd, proj - 1) - 0.5 * proj) / (double)as_cptr(A->cs)[t].x +
+                                  vol_x * 0.5 + 1.0);
+        float sum = 0.0f;
+        int cnt = 0;
+        if (d.y > 0) {
+            const cptr<float4> G = as_cptr(A->geo) + d.x;
+            if (!SENT && d.w != 0) {
+                fp_run<false, false>((const char*)band, rowb, G, d.y, d.z, tf1, xmax1, make_int2(0, 0),
+                                     sum, cnt);
+            } else {
+                int2 rr = make_int2(0, 0);
+                if (xd < proj) rr = ldgo(as_gptr(A->fp_range) + (size_t)t * proj + xd);
+                fp_run<true, SENT>((const char*)band, rowb, G, d.y, d.z, tf1, xmax1, rr, sum, cnt);
+            }
+        }
+        if (xd < proj) {
+            part[j * A->stride + xd] = sum;
+            if (SENT) part_n[j * A->stride + xd] = (uint16_t)cnt;
+        }
+    }
+}
+
+__global__ __launch_bounds__(FP_THREADS) void k_fp_part(const FpArgs* __restrict__ a, int slot_step)
+{
+    extern __shared__ float2 band[];
+    const cptr<FpArgs> A = as_cptr(a);
+    const int y = blockIdx.y, b = blockIdx.z / slot_step, slot0 = blockIdx.z - b * slot_step;
+    if (as_cptr(A->vflag)[y] != 0)
+        fp_part_band<true>(A, band, blockIdx.x, y, gridDim.y, b, slot0, slot_step);
+    else
+        fp_part_band<false>(A, band, blockIdx.x, y, gridDim.y, b, slot0, slot_step);
+}
+
+template <typename S>
+__global__ __launch_bounds__(256) void k_fp_sum(const FpArgs* __restrict__ a)
+{
+    const cptr<FpArgs> A = as_cptr(a);
+    const int xd = blockIdx.x * 256 + threadIdx.x, j = blockIdx.y, y = blockIdx.z, vol_y = gridDim.z;
+    const int nb = A->nb, proj = A->proj, stride = A->stride;
+    if (xd >= proj) return;
+    const int t = as_cptr(A->fp_list)[j], gx = j / A->group;
+    const bool sent = as_cptr(A->vflag)[y] != 0;
+    const size_t pitch = (size_t)vol_y * A->diff_rows * stride;   // a band's sums
+    const size_t at = ((size_t)y * A->diff_rows + j) * stride + xd;
+    const gptr<const float> part = as_gptr((const float*)A->part) + at;
+    const gptr<const uint16_t> part_n = (gptr<const uint16_t>)(as_gptr((const float*)A->part) + nb * pitch) + at;
+    const int rot = (int)(((unsigned)y * 5u + (unsigned)gx) % (unsigned)nb);   // as in fp_block
+    float acc = 0.0f;
+    int cnt = 0;
+#pragma unroll 8
+    for (int bi = 0; bi < nb; bi++) {
+        const int b = bi + rot < nb ? bi + rot : bi + rot - nb;
+        acc += part[b * pitch];
+    }
+    if (sent)
+        for (int b = 0; b < nb; b++) cnt += part_n[b * pitch];
+    const int count = sent ? cnt : as_gptr(A->fp_range)[(size_t)t * proj + xd].y;
+    fp_store_diff<S>(A, y, j, t, xd, acc, count);
 }
 
 // Forward projection + difference of many series in persistent launches:
@@ -516,6 +629,7 @@ FpArgs fp_args(const Plan& p, const int* fp_list, int n_list, const int* sched)
     a.stride = p.sino_stride;
     a.diff = p.d_diff;
     a.diff_rows = p.max_subset;
+    a.part = p.d_fp_part;
     return a;
 }
 
@@ -528,6 +642,21 @@ size_t fp_lds_bytes(int bz, int vol_x, int pf)
     const size_t pairs = fp_pair_bytes(bz, vol_x);
     if (pf != FP_PF_DMA) return pairs;
     return (pairs + 255) / 256 * 256 + (size_t)(bz + 1) * vol_x * sizeof(float);
+}
+
+// Scratch of the projector for few slices (k_fp_part) with n_bands bands of bz
+// rows, 0 where fp_block is used.  Counts of samples are 16 bits: a ray has at
+// most 1.5 max(VolX, bz) in a band, and VolX < 9600 (two rows of a band fit the
+// LDS).
+size_t fp_part_bytes(const Plan& p, int n_bands, int bz)
+{
+    const int group = fp_group(p.proj, p.max_subset, fp_waves(p.fp_pf));
+    const int items = p.vol_y * ((p.max_subset + group - 1) / group);
+    const bool two = fp_pair_bytes(bz, p.vol_x) <= (size_t)FP_LDS_TWO;
+    if (p.queued || n_bands < 2 || items > (two ? FP_SPLIT_ITEMS_TWO : FP_SPLIT_ITEMS)) return 0;
+    const size_t bytes = (sizeof(float) + sizeof(uint16_t)) * n_bands * p.vol_y * p.max_subset *
+                         p.sino_stride;
+    return bytes <= FP_SPLIT_BYTES ? bytes : 0;
 }
 
 // Kernels with more than 64 KiB of dynamic LDS must say so once per device;
@@ -563,6 +692,18 @@ static void launch_fp_t(const Plan& p, int subset, hipStream_t s)
     dim3 grid((n_list + group - 1) / group, p.vol_y);
     const size_t shm = fp_lds_bytes(p.geo.fp_bz, p.vol_x, p.fp_pf);
     const FpArgs* a = p.d_fp_args + subset;
+    if (p.d_fp_part) {
+        // shares of the pair slots while the launch has less than a workgroup per CU
+        const int items = std::max(1, (int)(grid.x * grid.y) * p.geo.fp_nbands);
+        const int shares = std::max(1, std::min(FP_SPLIT_SHARES, FP_SPLIT_GROUPS / items));
+        const size_t bytes = fp_pair_bytes(p.geo.fp_bz, p.vol_x);
+        static std::atomic<unsigned long long> done{0};
+        allow_big_lds(k_fp_part, done);
+        hipLaunchKernelGGL(k_fp_part, dim3(grid.x, grid.y, p.geo.fp_nbands * shares), dim3(FP_THREADS),
+                           bytes, s, a, shares);
+        hipLaunchKernelGGL(k_fp_sum<S>, dim3((p.proj + 255) / 256, n_list, p.vol_y), dim3(256), 0, s, a);
+        return;
+    }
     // the sentinel-free slices (nearly all) take a variant with the band
     // pitch fixed at compile time for the common widths
     if (p.fp_pf == FP_PF_REG) {   // VolX 1024 or 2048

@@ -299,6 +299,7 @@ static atr_status admit(atr_server* s, Request& r)
 {
     atr_status st;
     r.sart->alloc = s->arena.get();
+    r.sart->queued = true;
     if ((st = plan_upload(*r.sart)) != ATR_OK) return st;
     if (r.wbp) {
         r.wbp->alloc = s->arena.get();
