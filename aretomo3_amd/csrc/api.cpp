@@ -244,8 +244,8 @@ static size_t plan_bytes_estimate(const Plan& p)
         b += vox * 4 + (size_t)p.vol_y * p.max_subset * p.sino_stride * sb;
         b += n * p.vol_z * 8 + n * p.proj * 8 + (size_t)p.vol_x * p.vol_z * 4;
         b += n * (size_t)(p.vol_z * 2.5 + 16) * 16;  // FP sample tables (bounded by 60 deg)
-        const int bz = fp_balanced_rows(fp_band_rows(p.vol_x), p.vol_z);
-        b += fp_part_bytes(p, (p.vol_z - 1 + bz - 1) / bz, bz);
+        const int bz = fp_default_rows(p.vol_x, p.vol_z, p.storage, fp_items(p));
+        b += fp_part_bytes(p, (p.vol_z - 1 + bz - 1) / bz);
         // back-projection tiles: every tilt is in the initial list and in a subset's
         const int kind = bp_kind_of(p.storage);
         b += 2 * n * (size_t)bp_ztiles(p.vol_z, 8, kind) * bp_xtiles(p.vol_x, kind) * BP_WAVES * sizeof(int2);
@@ -323,7 +323,7 @@ static atr_status sart_tables_device(Plan& p)
     if ((st = reupload(p, &p.d_fp_geo, g.fp_geo, B, p.tab_bytes[4])) != ATR_OK) return st;
     if ((st = reupload(p, &p.d_fp_desc, g.fp_desc, B, p.tab_bytes[5])) != ATR_OK) return st;
     if ((st = reupload(p, &p.d_fp_pairs, p.host.sched, B, p.tab_bytes[6])) != ATR_OK) return st;
-    const size_t part = fp_part_bytes(p, g.fp_nbands, g.fp_bz);
+    const size_t part = fp_part_bytes(p, g.fp_nbands);
     if (part != p.fp_part_alloc) {
         if (p.d_fp_part) {
             plan_mfree(p, p.d_fp_part);
@@ -418,12 +418,8 @@ static atr_status plan_host(Plan& p)
         // (2-5 % less than 16 tilts a stage at 5 to 6 tilts, 3 % more at 12)
         p.bp_tz = bp_default_tz(p.vol_x, p.vol_y, p.vol_z, bp_kind_of(p.storage));
         p.bp_chunk = p.max_subset <= 8 ? 8 : 16;
-        // default forward-projector staging: register prefetch where it is
-        // built (VolX 1024, 2048: measured faster at the full band height),
-        // else direct
-        return sart_tables_host(p, p.bp_tz, p.bp_chunk,
-                                fp_balanced_rows(fp_band_rows(p.vol_x), p.vol_z),
-                                fp_rp_supported(p.vol_x) ? FP_PF_REG : 0);
+        const int bz = fp_default_rows(p.vol_x, p.vol_z, p.storage, fp_items(p));
+        return sart_tables_host(p, p.bp_tz, p.bp_chunk, bz, fp_default_mode(p.vol_x, bz));
     }
     build_wbp_intervals(g.cos_sin, p.n, p.vol_x, p.vol_z, p.proj, g.wbp_lohi);
     // 2x-grid back-projection: tile windows/classes (excluded tilts are left
@@ -814,6 +810,8 @@ static atr_status plan_autotune(Plan& p, hipStream_t s, int* tz_out, int* chunk_
         // then those of the band-prefetching one where VolX allows it
         std::vector<std::pair<int, int>> fps;
         for (int bz : bzs) fps.push_back({bz, 0});
+        const int def = fp_default_rows(p.vol_x, p.vol_z, p.storage, fp_items(p));
+        if (std::find(bzs.begin(), bzs.end(), def) == bzs.end()) fps.push_back({def, 0});
         if (fp_pf_supported(p.vol_x)) {
             std::vector<int> pfz;
             fp_band_candidates(p.vol_x, p.vol_z, pfz, FP_PF_DMA);

@@ -82,12 +82,12 @@ constexpr int FP_RP_ISSUE = 8;                // register prefetch: pair slots b
 // Few (slice, tilt group) items: up to this many, the bands of a slice are
 // projected side by side (k_fp_part, k_fp_sum).  Measured per pass (4
 // iterations, 5 subsets of 41 tilts), bands in turn / side by side:
-// 1024 x 8 x 256 (items 8) 4.05 / 0.68 ms, 1024 x 128 5.67 / 4.95, 1024 x 256
+// 1024 x 8 x 256 (8 items) 4.05 / 0.68 ms, 1024 x 128 5.67 / 4.95, 1024 x 256
 // 6.97 / 9.77; 700 x 100 x 300 4.93 / 3.48, 700 x 200 5.84 / 6.55.  Where two
 // workgroups' bands fit the LDS of a CU the line lies higher: 512 x 256 x 128
 // 2.41 / 2.19, 300 x 300 x 100 2.41 / 1.77.
 constexpr int FP_SPLIT_ITEMS = 128, FP_SPLIT_ITEMS_TWO = 384;
-constexpr int FP_LDS_TWO = 80 * 1024;         // bands of which two fit the LDS
+constexpr int FP_LDS_TWO = 80 * 1024 - 256;   // bands of which two fit the LDS (and the queue's word)
 constexpr size_t FP_SPLIT_BYTES = 256 << 20;  // the bands' sums at most
 // workgroups up to which a band's pair slots are shared out, and shares
 constexpr int FP_SPLIT_GROUPS = 256, FP_SPLIT_SHARES = 4;
@@ -393,7 +393,8 @@ struct FpItem {
 // staging (VolX 512, 1024, 2048, any), 8-9: register prefetch (VolX 1024,
 // 2048).
 constexpr int FP_VARIANT_EMPTY = 10;
-constexpr int FP_VARIANTS = 11;
+constexpr int FP_VARIANT_ANY = 11;
+constexpr int FP_VARIANTS = 12;
 int fp_variant(const FpArgs& a);
 struct FpLaunch {
     int first;       // first entry of its queue in the item array
@@ -475,6 +476,8 @@ bool build_fp_tables(const std::vector<float>& cs, int n, int vol_x, int vol_z, 
                      int bz, Geometry& g);
 int fp_band_rows(int vol_x, int pf = 0);
 int fp_balanced_rows(int bz_max, int vol_z);
+int fp_default_rows(int vol_x, int vol_z, int storage, int items);
+int fp_default_mode(int vol_x, int bz);
 void fp_band_candidates(int vol_x, int vol_z, std::vector<int>& rows, int pf = 0);
 int fp_group(int proj, int n_list, int n_waves = FP_WAVES);
 // fn(0) .. fn(n - 1) on up to 16 host threads (returns when all are done).
@@ -507,7 +510,8 @@ size_t spec_elems(int columns, int rows, int kb);
 // first: offset of the list in p.d_lists
 BpArgs bp_args(const Plan& p, const void* sino, int rows, int first, int n_list, float relax,
                bool check_sent);
-size_t fp_part_bytes(const Plan& p, int n_bands, int bz);
+int fp_items(const Plan& p);   // (slice, tilt group) items of the largest subset
+size_t fp_part_bytes(const Plan& p, int n_bands);
 FpArgs fp_args(const Plan& p, const int* fp_list, int n_list, const int* sched);
 size_t fp_lds_bytes(int bz, int vol_x, int pf = 0);
 // step 0: initial back-projection, 1 + s: subset s (arguments in p.d_bp_args)

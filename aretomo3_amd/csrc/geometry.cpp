@@ -462,6 +462,40 @@ int fp_balanced_rows(int bz_max, int vol_z)
     return (cells + nb - 1) / nb;
 }
 
+// Cell rows per band that a plan starts with: the largest of which two
+// workgroups' bands fit the LDS, if that is at least 8 (VolX up to 1134), else
+// the largest that fits.  One workgroup samples while the other waits for its
+// band; per launch of 41 tilts in 5 subsets, one / two workgroups per CU:
+// 700 x 700 x 200 0.420 / 0.341 ms (17 / 13 rows), 900 x 600 x 256 0.647 /
+// 0.561 (10 rows), 1000 x 520 x 300 0.796 / 0.716 (9), 1024 x 1024 x 256 0.845
+// (register prefetch) / 0.814 (8); 512 x 512 x 128 (17 rows in both) 0.21 /
+// 0.17.  Lower bands lose to their reloads (1024 with 7 rows: 0.882).
+// With more items (slice, tilt group) than are projected side by side but no
+// more than CUs there is one workgroup per CU anyway, and high bands are
+// better (1024 x 200 x 256: 0.214 ms, 0.293 with 8 rows; 900 x 250 x 256: 0.230,
+// 0.254 with 10).
+// With BF16 storage the bands stay as high as they fit: a ray's samples are
+// summed band by band, and the last bit of a sum decides the last of the 8 bits
+// that a difference keeps.
+static int fp_two_rows(int vol_x)
+{
+    const int rows = FP_LDS_TWO / ((vol_x + 1) * (int)sizeof(float2)) - 1;
+    return rows < 8 ? 0 : std::min(FP_BZ_MAX, rows);
+}
+int fp_default_rows(int vol_x, int vol_z, int storage, int items)
+{
+    const bool one = storage == ATR_STORAGE_BF16 || (items > FP_SPLIT_ITEMS && items <= 256);
+    const int two = one ? 0 : fp_two_rows(vol_x);
+    return fp_balanced_rows(two ? two : fp_band_rows(vol_x), vol_z);
+}
+// Staging that a plan starts with: direct with two workgroups per CU, else
+// register prefetch where it is built (VolX 1024, 2048), else direct.
+int fp_default_mode(int vol_x, int bz)
+{
+    if (fp_lds_bytes(bz, vol_x, 0) <= (size_t)FP_LDS_TWO) return 0;
+    return fp_rp_supported(vol_x) ? FP_PF_REG : 0;
+}
+
 // Band heights the autotuner times: the largest that fits the LDS, then
 // about 2/3 and 1/2 of it, each balanced over the slice's cell rows, none
 // above the LDS limit, no height twice.  At VolX >= 6400 only one row fits
@@ -506,6 +540,9 @@ void fp_pair_schedule(const Geometry& g, const int* list, int n_list, int proj, 
 {
     const int ntile = (proj + FP_WAVE - 1) / FP_WAVE;
     const int nb = g.fp_nbands;
+    // two workgroups per CU: one fills the other's waits, exchanges give less than
+    // 1 % there (and take a third of the plan's time)
+    const bool two = fp_lds_bytes(g.fp_bz, proj, 0) <= (size_t)FP_LDS_TWO;
     for (int j0 = 0; j0 < n_list; j0 += group) {
         const int ng = std::min(group, n_list - j0);
         const int n_items = ng * ntile;
@@ -589,7 +626,8 @@ void fp_pair_schedule(const Geometry& g, const int* list, int n_list, int proj, 
             }
         };
         for (int b = 0; b < nb; b++) rank_band(b);
-        for (int pass = 0; pass < 4; pass++) {
+        const int passes = two ? 0 : 4;
+        for (int pass = 0; pass < passes; pass++) {
             bool improved = false;
             for (int a = 0; a < n_items; a++)
                 for (int c = a + 1; c < n_items; c++) {

@@ -441,12 +441,19 @@ __device__ __forceinline__ void fp_block(cptr<FpArgs> A, float2* __restrict__ ba
     }
 }
 
+// Waves per SIMD that a kernel is built for: 8 (two workgroups per CU, at most 64
+// VGPRs) where the bands of two workgroups fit the LDS, so that one samples while
+// the other waits at its band's barriers.  A few values spill outside the sample
+// loops, which costs 2 % where only one workgroup is on a CU.
+constexpr int fp_waves_per_simd(bool two) { return two ? 8 : 4; }
+
 // ROWB: the band row pitch in bytes, 8 (VolX + 1), when the launch fixes it
 // at compile time (VolX 512, 1024, 2048), else 0.
 // PF: the band-prefetching variant (VolX a multiple of 256).
 // RP: the register-prefetching variant (columns per thread).
-template <typename S, bool SENT, int ROWB, bool PF = false, int RP = 0>
-__global__ __launch_bounds__(FP_THREADS) void k_for_proj_diff(const FpArgs* __restrict__ a)
+// TWO: two workgroups per CU.
+template <typename S, bool SENT, int ROWB, bool PF = false, int RP = 0, bool TWO = false>
+__global__ __launch_bounds__(FP_THREADS, fp_waves_per_simd(TWO)) void k_for_proj_diff(const FpArgs* __restrict__ a)
 {
     extern __shared__ float2 band[];
     // slices from the last to the first, the back-projections run from the
@@ -464,8 +471,8 @@ __global__ __launch_bounds__(FP_THREADS) void k_for_proj_diff(const FpArgs* __re
 // bits.  Slices with and without empty voxels go through one launch.
 //
 // fp_block walks the bands of a slice one after the other: with one slice of
-// 512 x 128 that is one busy CU, and 65 us for 8 tilts of 512 rays, of which
-// the samples are 4; with the bands side by side the two launches take FPP_US.
+// 512 x 128 that is one busy CU, and 65 us for 8 tilts of 512 rays; with the
+// bands side by side the two launches take 7.5 and 3.1 us.
 // ------------------------------------------------------------------------
 template <bool SENT>
 __device__ __forceinline__ void fp_part_band(cptr<FpArgs> A, float2* __restrict__ band, int gx, int y,
@@ -575,16 +582,16 @@ template <typename S, int V>
 __device__ __forceinline__ void fp_variant_block(cptr<FpArgs> A, float2* band, int gx, int y)
 {
     // VolX class: 0: 512, 1: 1024, 2: 2048, 3: any (pitch at run time)
-    constexpr int W = V < 8 ? V % 4 : V - 7;
+    constexpr int W = V < 8 ? V % 4 : V == FP_VARIANT_ANY ? 3 : V - 7;
     constexpr int ROWB = W == 0 ? 513 * 8 : W == 1 ? 1025 * 8 : W == 2 ? 2049 * 8 : 0;
     if constexpr (V == FP_VARIANT_EMPTY) fp_block<S, true>(A, band, gx, y);
     else if constexpr (V < 4) fp_block<S, false, ROWB, true>(A, band, gx, y);
-    else if constexpr (V < 8) fp_block<S, false, ROWB>(A, band, gx, y);
+    else if constexpr (V < 8 || V == FP_VARIANT_ANY) fp_block<S, false, ROWB>(A, band, gx, y);
     else fp_block<S, false, ROWB, false, W>(A, band, gx, y);   // RP: 1 or 2 columns
 }
 
 template <typename S, int V>
-__global__ __launch_bounds__(FP_THREADS) void k_for_proj_diff_batch(const FpItem* __restrict__ e,
+__global__ __launch_bounds__(FP_THREADS, fp_waves_per_simd(V == 4 || V == 5 || V == 7)) void k_for_proj_diff_batch(const FpItem* __restrict__ e,
                                                                    int n_e, int total,
                                                                    int* __restrict__ counter)
 {
@@ -644,16 +651,19 @@ size_t fp_lds_bytes(int bz, int vol_x, int pf)
     return (pairs + 255) / 256 * 256 + (size_t)(bz + 1) * vol_x * sizeof(float);
 }
 
-// Scratch of the projector for few slices (k_fp_part) with n_bands bands of bz
-// rows, 0 where fp_block is used.  Counts of samples are 16 bits: a ray has at
-// most 1.5 max(VolX, bz) in a band, and VolX < 9600 (two rows of a band fit the
-// LDS).
-size_t fp_part_bytes(const Plan& p, int n_bands, int bz)
+int fp_items(const Plan& p)
 {
     const int group = fp_group(p.proj, p.max_subset, fp_waves(p.fp_pf));
-    const int items = p.vol_y * ((p.max_subset + group - 1) / group);
-    const bool two = fp_pair_bytes(bz, p.vol_x) <= (size_t)FP_LDS_TWO;
-    if (p.queued || n_bands < 2 || items > (two ? FP_SPLIT_ITEMS_TWO : FP_SPLIT_ITEMS)) return 0;
+    return p.vol_y * ((p.max_subset + group - 1) / group);
+}
+
+// Scratch of the projector for few slices (k_fp_part) with n_bands bands, 0 where fp_block is used.  Counts of samples are 16 bits: a ray has at
+// most 1.5 max(VolX, bz) in a band, and VolX < 9600 (two rows of a band fit the
+// LDS).
+size_t fp_part_bytes(const Plan& p, int n_bands)
+{
+    const bool two = fp_pair_bytes(FP_BZ_MAX, p.vol_x) <= (size_t)FP_LDS_TWO;   // VolX <= 566
+    if (p.queued || n_bands < 2 || fp_items(p) > (two ? FP_SPLIT_ITEMS_TWO : FP_SPLIT_ITEMS)) return 0;
     const size_t bytes = (sizeof(float) + sizeof(uint16_t)) * n_bands * p.vol_y * p.max_subset *
                          p.sino_stride;
     return bytes <= FP_SPLIT_BYTES ? bytes : 0;
@@ -676,12 +686,12 @@ static void allow_big_lds(K kernel, std::atomic<unsigned long long>& done, int b
     if (e != hipSuccess) (void)hipGetLastError();
 }
 
-template <typename S, bool SENT, int ROWB, bool PF = false, int RP = 0>
+template <typename S, bool SENT, int ROWB, bool PF = false, int RP = 0, bool TWO = false>
 static void launch_fp_k(dim3 grid, size_t shm, const FpArgs* a, hipStream_t s)
 {
     static std::atomic<unsigned long long> done{0};
-    allow_big_lds(k_for_proj_diff<S, SENT, ROWB, PF, RP>, done, PF ? FP_LDS_PF : FP_LDS_BUDGET);
-    hipLaunchKernelGGL((k_for_proj_diff<S, SENT, ROWB, PF, RP>), grid, dim3(FP_THREADS), shm, s, a);
+    allow_big_lds(k_for_proj_diff<S, SENT, ROWB, PF, RP, TWO>, done, PF ? FP_LDS_PF : FP_LDS_BUDGET);
+    hipLaunchKernelGGL((k_for_proj_diff<S, SENT, ROWB, PF, RP, TWO>), grid, dim3(FP_THREADS), shm, s, a);
 }
 
 template <typename S>
@@ -722,11 +732,18 @@ static void launch_fp_t(const Plan& p, int subset, hipStream_t s)
         launch_fp_k<S, true, 0, true>(grid, shm, a, s);
         return;
     }
-    switch (p.vol_x) {
-    case 512: launch_fp_k<S, false, 513 * 8>(grid, shm, a, s); break;
-    case 1024: launch_fp_k<S, false, 1025 * 8>(grid, shm, a, s); break;
-    case 2048: launch_fp_k<S, false, 2049 * 8>(grid, shm, a, s); break;
-    default: launch_fp_k<S, false, 0>(grid, shm, a, s); break;
+    if (shm <= (size_t)FP_LDS_TWO) {
+        switch (p.vol_x) {
+        case 512: launch_fp_k<S, false, 513 * 8, false, 0, true>(grid, shm, a, s); break;
+        case 1024: launch_fp_k<S, false, 1025 * 8, false, 0, true>(grid, shm, a, s); break;
+        default: launch_fp_k<S, false, 0, false, 0, true>(grid, shm, a, s); break;
+        }
+    } else {
+        switch (p.vol_x) {
+        case 1024: launch_fp_k<S, false, 1025 * 8>(grid, shm, a, s); break;
+        case 2048: launch_fp_k<S, false, 2049 * 8>(grid, shm, a, s); break;
+        default: launch_fp_k<S, false, 0>(grid, shm, a, s); break;
+        }
     }
     launch_fp_k<S, true, 0>(grid, shm, a, s);
 }
@@ -738,13 +755,16 @@ void launch_fp_diff(const Plan& p, int subset, hipStream_t s)
     else launch_fp_t<float>(p, subset, s);
 }
 
-// Staging variant of a series' plan (slices without empty voxels).
+// Staging variant of a series' plan (slices without empty voxels): 0-3 DMA, 4, 5, 7
+// direct with two workgroups per CU (VolX 512, 1024, any), 6 and FP_VARIANT_ANY
+// direct with one (VolX 2048, any), 8-9 registers.
 int fp_variant(const FpArgs& a)
 {
     const int w = a.vol_x == 512 ? 0 : a.vol_x == 1024 ? 1 : a.vol_x == 2048 ? 2 : 3;
     if (a.pf == FP_PF_DMA) return w;
     if (a.pf == FP_PF_REG && (w == 1 || w == 2)) return 7 + w;
-    return 4 + w;
+    if (fp_pair_bytes(a.bz, a.vol_x) <= (size_t)FP_LDS_TWO) return w == 2 ? 7 : 4 + w;
+    return w == 2 ? 6 : FP_VARIANT_ANY;
 }
 
 std::vector<FpLaunch> lay_out_fp(const std::vector<QueueEntry<FpItem>>& ent, FpItem* out)

@@ -2,7 +2,9 @@
 sums added afterwards) against the FP64 oracle and, bit for bit, against the
 one that walks the bands in turn, which batches run: one to 40 slices, widths
 beside the 64-ray tiles, two groups of tilts, one band row, steep tilts, slices
-with empty voxels."""
+with empty voxels.  And the bands-in-turn projector where two of its workgroups
+share a CU: more items than CUs, the widest slice whose bands of 8 rows fit
+twice and the next."""
 import numpy as np
 import pytest
 
@@ -40,6 +42,26 @@ def test_few_slices(gpu_available, px, py, vol_z, n, subsets, rows, storage, tol
     ref = oracle.recon_slices(proj.astype(np.float64), tilts, 1, vol_z, list(range(py)), iters=2,
                               n_subsets=subsets, relax=0.3, order=1, positivity=0)
     assert rel_l2(got, ref) <= tol
+
+
+@pytest.mark.parametrize("px,py,vol_z,storage,tol", [
+    (65, 400, 30, L.STORAGE_F32, 1e-5), (512, 390, 20, L.STORAGE_F16, 2e-3),
+    (1024, 260, 30, L.STORAGE_F32, 1e-5), (1134, 260, 19, L.STORAGE_F32, 1e-5),
+    (1135, 260, 19, L.STORAGE_F32, 1e-5), (300, 390, 40, L.STORAGE_BF16, 8e-3),
+    (700, 200, 30, L.STORAGE_F32, 1e-5)])
+def test_two_workgroups_per_cu(gpu_available, px, py, vol_z, storage, tol):
+    tilts = np.linspace(-60.0, 66.0, 9).astype(np.float32)
+    proj, _ = phantom.tilt_series(px + py, px, py, tilts, vol_z, n_ellipsoids=30, axis_min=3,
+                                  axis_max=12, noise_frac=0.05)
+    print(f"case {px} x {py} x {vol_z}, storage {storage}", flush=True)
+    plan = Plan(px, py, tilts, vol_z, L.METHOD_SART, sart_iters=2, sart_subsets=2, relax=0.3,
+                subset_order=L.SUBSETS_INTERLEAVED, positivity=False, storage=storage)
+    got = plan.execute_host(proj)
+    assert np.array_equal(got, _in_batch(plan, proj))
+    rows = [0, 1, py // 2, py - 1]
+    ref = oracle.recon_slices(proj.astype(np.float64), tilts, 1, vol_z, rows, iters=2, n_subsets=2,
+                              relax=0.3, order=1, positivity=0)
+    assert rel_l2(got[rows], ref) <= tol
 
 
 def test_few_slices_with_empty_voxels(gpu_available):
