@@ -468,8 +468,8 @@ int fp_balanced_rows(int bz_max, int vol_z)
 // band; per launch of 41 tilts in 5 subsets, one / two workgroups per CU:
 // 700 x 700 x 200 0.420 / 0.341 ms (17 / 13 rows), 900 x 600 x 256 0.647 /
 // 0.561 (10 rows), 1000 x 520 x 300 0.796 / 0.716 (9), 1024 x 1024 x 256 0.845
-// (register prefetch) / 0.814 (8); 512 x 512 x 128 (17 rows in both) 0.21 /
-// 0.17.  Lower bands lose to their reloads (1024 with 7 rows: 0.882).
+// (register prefetch) / 0.814 (8); 512 x 512 x 128 (16 rows in both) 0.154 /
+// 0.117.  Lower bands lose to their reloads (1024 with 7 rows: 0.882).
 // With more items (slice, tilt group) than are projected side by side but no
 // more than CUs there is one workgroup per CU anyway, and high bands are
 // better (1024 x 200 x 256: 0.214 ms, 0.293 with 8 rows; 900 x 250 x 256: 0.230,

@@ -4,7 +4,7 @@
 //   k_wbp_rowfft    row FFT of two rows of the 2x grid (the back-projection
 //                   onto that grid is k_wbp_grid_bp in kernels_sart.hip)
 //                   (Recon/GBackProjWbp.cu:126)
-//   k_wbp_colfft    column FFT, normalisation, crop, inverse column FFT
+//   k_colfft        column FFT, normalisation, crop, inverse column FFT
 //                   (MaUtil/CCufft2D.cpp:65-80, MaUtil/GFourierResize2D.cu:7-39)
 //   k_wbp_rowc2r    real inverse row FFT + output layout
 //                   (MaUtil/CCufft2D.cpp:108-123, MaUtil/CPad2D.cpp:29-39,
@@ -102,7 +102,7 @@ __device__ __forceinline__ float2 spec_join(const float2* h, int k, int n, int r
 // bx x by (MaUtil/GFourierResize2D.cu:7-39), unnormalised C2R.
 //   k_bin_rowfft  two image rows packed as one complex row, FFT of length
 //                 ax, the columns kx < bx/2+1 of both half spectra kept
-//   k_bin_colfft  per block of columns: FFT of length ay, normalisation,
+//   k_colfft      per block of columns: FFT of length ay, normalisation,
 //                 crop to by rows, inverse FFT of length by
 //   k_bin_rowc2r  two binned rows: packed C2R of length bx
 // ------------------------------------------------------------------------
