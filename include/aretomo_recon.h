@@ -182,7 +182,8 @@ atr_status atr_plan_set_tile_shape(atr_plan* plan, int bp_tz, int bp_chunk, int 
                                    int fp_prefetch);
 /* The forward-projection band heights (cell rows) the autotuner times for a
  * slice of vol_x x vol_z, without a GPU: every one fits the LDS, none
- * appears twice.  *n receives their number (at most 3); rows may be NULL. */
+ * appears twice.  *n receives their number (at most 3); rows may be NULL.
+ * The autotuner also times the height that the plan starts with. */
 atr_status atr_fp_band_candidates(int vol_x, int vol_z, int* rows, int cap, int* n);
 atr_status atr_plan_set_profiling(atr_plan* plan, int enable);
 atr_status atr_plan_kernel_stats(const atr_plan* plan, int kernel, int* launches,
