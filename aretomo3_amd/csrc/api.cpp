@@ -354,9 +354,12 @@ static atr_status sart_tables_device(Plan& p)
     return ATR_OK;
 }
 
-// Rebuilds the shape-dependent tables (autotuner, atr_plan_set_tile_shape).
+// Rebuilds the shape-dependent tables (autotuner, atr_plan_set_tile_shape).  A
+// prefetching projector that is asked for is run, also where the slices are so
+// few that the bands would be projected side by side.
 static atr_status sart_tables(Plan& p, int tz, int chunk, int bz, int pf)
 {
+    p.fp_split = pf == 0;
     atr_status st = sart_tables_host(p, tz, chunk, bz, pf);
     if (st != ATR_OK) return st;
     return sart_tables_device(p);

@@ -270,6 +270,7 @@ struct Plan {
     FpArgs* d_fp_args = nullptr;      // per subset
     float* d_fp_part = nullptr;       // FpArgs::part; null: fp_block does it
     size_t fp_part_alloc = 0;
+    bool fp_split = true;             // few slices: bands side by side; off with a staging set by hand
     bool queued = false;              // only run in work-queue launches (serve)
     float* d_wbp_grid = nullptr;      // [slab][2VolZ][2VolX] the 2x-grid back-projection
     int2* d_wbp_tiles = nullptr;      // the 2x grid's, as bp_tiles

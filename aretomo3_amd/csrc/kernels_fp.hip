@@ -657,13 +657,13 @@ int fp_items(const Plan& p)
     return p.vol_y * ((p.max_subset + group - 1) / group);
 }
 
-// Scratch of the projector for few slices (k_fp_part) with n_bands bands, 0 where fp_block is used.  Counts of samples are 16 bits: a ray has at
-// most 1.5 max(VolX, bz) in a band, and VolX < 9600 (two rows of a band fit the
-// LDS).
+// Scratch of the projector for few slices (k_fp_part) with n_bands bands, 0 where
+// fp_block is used.  Counts of samples are 16 bits: a ray has at most 1.5
+// max(VolX, bz) in a band, and VolX < 9600 (two rows of a band fit the LDS).
 size_t fp_part_bytes(const Plan& p, int n_bands)
 {
     const bool two = fp_pair_bytes(FP_BZ_MAX, p.vol_x) <= (size_t)FP_LDS_TWO;   // VolX <= 566
-    if (p.queued || n_bands < 2 || fp_items(p) > (two ? FP_SPLIT_ITEMS_TWO : FP_SPLIT_ITEMS)) return 0;
+    if (p.queued || !p.fp_split || n_bands < 2 || fp_items(p) > (two ? FP_SPLIT_ITEMS_TWO : FP_SPLIT_ITEMS)) return 0;
     const size_t bytes = (sizeof(float) + sizeof(uint16_t)) * n_bands * p.vol_y * p.max_subset *
                          p.sino_stride;
     return bytes <= FP_SPLIT_BYTES ? bytes : 0;

@@ -176,8 +176,10 @@ atr_status atr_plan_autotune(atr_plan* plan, void* stream, int* bp_tz, int* bp_c
                              int* fp_band_rows, int* fp_prefetch);
 /* Sets the tile shapes by hand: bp_tz, bp_chunk in {8, 16}; fp_prefetch 0, 1
  * (VolX a multiple of 256) or 2 (VolX 1024 or 2048); fp_band_rows in
- * [1, the largest band that fits in LDS for that forward projector].  Refused for a plan that
- * belongs to a batch, as atr_plan_autotune. */
+ * [1, the largest band that fits in LDS for that forward projector].  With
+ * fp_prefetch 1 or 2 that projector runs whatever the number of slices; with 0
+ * the bands of few slices are projected side by side (the same result).
+ * Refused for a plan that belongs to a batch, as atr_plan_autotune. */
 atr_status atr_plan_set_tile_shape(atr_plan* plan, int bp_tz, int bp_chunk, int fp_band_rows,
                                    int fp_prefetch);
 /* The forward-projection band heights (cell rows) the autotuner times for a
