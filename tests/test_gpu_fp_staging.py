@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 import oracle
-from aretomo3_amd import DeviceArray, Plan, phantom, synchronize
+from aretomo3_amd import Batch, DeviceArray, Plan, phantom, synchronize
 from aretomo3_amd import _lib as L
 from helpers import rel_l2
 
@@ -134,3 +134,41 @@ def test_few_slices_and_staging_set_by_hand(gpu_available, px, vol_z, rows, mode
     plan.set_tile_shape(16, 16, rows)
     assert plan.device_bytes == size
     plan.close()
+
+
+@pytest.mark.parametrize("storage", [L.STORAGE_F32, L.STORAGE_BF16])
+def test_batch_with_empty_voxels(gpu_available, storage):
+    """Voxels that become empty during the iterations (one projection value far
+    below the others, one tilt a subset, relaxation 1.5: a step of -1.3e10), in
+    slices 0 and 2: a batch, whose launch for slices with empty voxels they
+    take, gives what the plan gives alone, bands side by side and in turn."""
+    px, py, vol_z, n = 256, 4, 36, 7
+    tilts = np.linspace(-46.0, 53.0, n).astype(np.float32)
+    proj, _ = phantom.tilt_series(9, px, py, tilts, vol_z, n_ellipsoids=30, axis_min=3, axis_max=12,
+                                  noise_frac=0.05)
+    proj[3, [0, 2], 30:50] = -9e9 * vol_z / np.cos(np.deg2rad(tilts[3]))
+    # a fill table that maps each voxel to itself fills with the slice's mean:
+    # many equal values show that the slice had empty voxels
+    for y in range(py):
+        sino = np.zeros((n, px + 2))
+        sino[:, :px] = proj[:, y]
+        ref, _ = oracle.tomo_sart(sino, px, oracle.cos_sin(tilts), np.zeros((vol_z, px)), 0, n, 1, n,
+                                  relax=1.5, positivity=0, fill_tbl=np.arange(vol_z * px))
+        assert (np.unique(ref, return_counts=True)[1].max() > 300) == (y in (0, 2))
+    print(f"case batch with empty voxels, storage {storage}", flush=True)
+    kw = dict(sart_iters=3, sart_subsets=n, relax=1.5, positivity=False, fill_seed=3, storage=storage)
+    plan = Plan(px, py, tilts, vol_z, L.METHOD_SART, **kw)
+    other = Plan(px, 2, tilts, 20, L.METHOD_SART, **kw)
+    for pf in (0, 1):
+        plan.set_tile_shape(16, 16, 8, pf)
+        alone = plan.execute_host(proj)
+        d_in, d_in2 = DeviceArray.from_numpy(proj), DeviceArray.from_numpy(proj[:, [1, 3]])
+        d_out = [DeviceArray(4 * int(np.prod(p.volume_shape))) for p in (plan, other)]
+        batch = Batch([plan, other])
+        batch.execute([d_in, d_in2], d_out)
+        synchronize()
+        assert np.array_equal(d_out[0].to_numpy(plan.volume_shape), alone), pf
+        batch.close()
+        if pf == 0:
+            first = alone
+    assert np.array_equal(alone, first)
