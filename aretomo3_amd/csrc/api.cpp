@@ -722,13 +722,15 @@ atr_status plan_execute(Plan& p, const float* in, float* out, int accumulate, hi
 // Times the candidate tile shapes on the plan's own geometry and keeps the
 // fastest: back-projection z rows per thread x tilts per LDS stage, then
 // forward-projection band rows.  Choices are cached per (sizes, tilts,
-// subsets, storage), so later plans of the same shape skip the timing.
+// subsets, storage), so later plans of the same shape skip the timing.  The
+// number of slices is one of the sizes: it decides whether the bands go side by
+// side, how many workgroups share a CU and how well tiles fill the chip.
 struct TuneKey {
-    int vol_x, vol_z, proj, n, n_subsets, storage;
+    int vol_x, vol_y, vol_z, proj, n, n_subsets, storage;
     bool operator<(const TuneKey& o) const
     {
-        return std::tie(vol_x, vol_z, proj, n, n_subsets, storage) <
-               std::tie(o.vol_x, o.vol_z, o.proj, o.n, o.n_subsets, o.storage);
+        return std::tie(vol_x, vol_y, vol_z, proj, n, n_subsets, storage) <
+               std::tie(o.vol_x, o.vol_y, o.vol_z, o.proj, o.n, o.n_subsets, o.storage);
     }
 };
 struct TuneChoice {
@@ -768,7 +770,7 @@ static atr_status plan_autotune(Plan& p, hipStream_t s, int* tz_out, int* chunk_
     if (p.batch_refs > 0)
         return fail(ATR_ERR_INVALID_ARG,
                     "autotune: the plan belongs to a batch (destroy the batch first)");
-    const TuneKey key{p.vol_x, p.vol_z, p.proj, p.n, p.n_subsets, p.storage};
+    const TuneKey key{p.vol_x, p.vol_y, p.vol_z, p.proj, p.n, p.n_subsets, p.storage};
     TuneChoice best{p.bp_tz, p.bp_chunk, p.geo.fp_bz, p.fp_pf};
     bool cached = false;
     {

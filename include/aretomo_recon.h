@@ -164,7 +164,8 @@ atr_status atr_execute_host(atr_plan* plan, const float* proj_host, float* vol_h
  * wave streams the next z-band into LDS while the others sample) and (VolX
  * 1024, 2048) the register-prefetching one (fp_prefetch = 2: every
  * thread loads its columns of the next z-band into registers while the band
- * is sampled) -- and keeps the fastest.  Choices are cached per shape within the process.  Every voxel
+ * is sampled) -- and keeps the fastest.  Choices are cached within the process
+ * per shape (volume, projections, subsets, storage).  Every voxel
  * sums its tilts in the same order whatever the shape; the FP32 rounding of
  * the back-projection coordinate (taken relative to the tile's window) and
  * the order in which a forward ray adds up its z-bands depend on the shape,
