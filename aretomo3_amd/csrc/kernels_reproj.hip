@@ -36,6 +36,34 @@ constexpr int RP_WAVES = 4;
 constexpr int RP_LDS = 52 * 1024;      // three workgroups per CU
 constexpr int RP_LDS_MAX = 150 * 1024;
 
+// The four waves' sums and counts of a ray, added in the ray's order, to its
+// output pixel.
+__device__ __forceinline__ void reproj_store(const ReprojArgs& a, const double (&sum)[RP_ROWS],
+                                             const int (&cnt)[RP_ROWS], double* s_sum, int y0, int x,
+                                             float* __restrict__ out)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int* s_cnt = (int*)(s_sum + RP_WAVES * RP_ROWS * 64);
+#pragma unroll
+    for (int r = 0; r < RP_ROWS; r++) {
+        s_sum[(wave * RP_ROWS + r) * 64 + lane] = sum[r];
+        s_cnt[(wave * RP_ROWS + r) * 64 + lane] = cnt[r];
+    }
+    __syncthreads();
+    const int n_rows = min(RP_ROWS, a.proj_y - y0);
+    for (int r = wave; r < n_rows; r += RP_WAVES) {
+        double t = 0.0;
+        int n = 0;
+        for (int w = 0; w < RP_WAVES; w++) {
+            t += s_sum[(w * RP_ROWS + r) * 64 + lane];
+            n += s_cnt[(w * RP_ROWS + r) * 64 + lane];
+        }
+        if (x < a.proj_x)
+            out[(size_t)(y0 + r) * a.proj_x + x] = ((float)n < a.min_count) ? kSentinel : (float)(t / n);
+    }
+}
+constexpr int RP_SUMS = RP_WAVES * RP_ROWS * 64 * (int)(sizeof(double) + sizeof(int));
+
 // N: number of reference tilts (their geometry stays in scalar registers).
 template <int N>
 __global__ __launch_bounds__(64 * RP_WAVES) void k_reproj(const float* __restrict__ projs,
@@ -48,7 +76,6 @@ __global__ __launch_bounds__(64 * RP_WAVES) void k_reproj(const float* __restric
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int xb = blockIdx.x * 64, x = xb + lane;
     const int y0 = blockIdx.y * RP_ROWS;
-    const int n_rows = min(RP_ROWS, a.proj_y - y0);
     const double fc = a.ray_cos, fs = a.ray_sin;
     const double hx = a.vol_x * 0.5, hz = a.vol_z * 0.5, cx = a.proj_x * 0.5;
     const int last = a.proj_x - 1;
@@ -172,25 +199,69 @@ __global__ __launch_bounds__(64 * RP_WAVES) void k_reproj(const float* __restric
         }
         __syncthreads();
     }
-    // the four waves' sums of a ray, in the ray's order
-    double* s_sum = (double*)win;
-    int* s_cnt = (int*)(s_sum + RP_WAVES * RP_ROWS * 64);
+#pragma unroll
+    for (int r = 0; r < RP_ROWS; r++) cnt[r] += plain_cnt;
+    reproj_store(a, sum, cnt, (double*)win, y0, x, out);
+}
+
+// The same without staged columns, for references so far from the projection
+// that those of a single sample do not fit the LDS (lists that are not in the
+// order of the tilts: ten references, one of them some 80 degrees from a steep
+// projection, spread 64 columns over more than 480).  Every value is looked at for
+// being empty.
+__global__ __launch_bounds__(64 * RP_WAVES) void k_reproj_far(const float* __restrict__ projs,
+                                                              ReprojArgs a, float* __restrict__ out)
+{
+#pragma clang fp contract(off)
+    __shared__ double sums[RP_SUMS / sizeof(double)];
+    const int x = blockIdx.x * 64 + (threadIdx.x & 63), wave = threadIdx.x >> 6;
+    const int y0 = blockIdx.y * RP_ROWS;
+    const double fc = a.ray_cos, fs = a.ray_sin;
+    const double cx = a.proj_x * 0.5;
+    const int last = a.proj_x - 1;
+    const double xp = x + 0.5 - a.proj_x * 0.5;
+    const double tx = a.vol_x * 0.5 + a.ray * 0.5 * fs + xp / fc;
+    const double tz = a.vol_z * 0.5 - a.ray * 0.5 * fc;
+    double sum[RP_ROWS];
+    int cnt[RP_ROWS];
 #pragma unroll
     for (int r = 0; r < RP_ROWS; r++) {
-        s_sum[(wave * RP_ROWS + r) * 64 + lane] = sum[r];
-        s_cnt[(wave * RP_ROWS + r) * 64 + lane] = cnt[r] + plain_cnt;
+        sum[r] = 0.0;
+        cnt[r] = 0;
     }
-    __syncthreads();
-    for (int r = wave; r < n_rows; r += RP_WAVES) {
-        double t = 0.0;
-        int n = 0;
-        for (int w = 0; w < RP_WAVES; w++) {
-            t += s_sum[(w * RP_ROWS + r) * 64 + lane];
-            n += s_cnt[(w * RP_ROWS + r) * 64 + lane];
+    const int per = (a.ray + RP_WAVES - 1) / RP_WAVES;
+    const int ia = wave * per, ib = min(ia + per, a.ray);
+    for (int i = ia; i < ib; i++) {
+        const double px = tx - i * fs;
+        const double pz = tz + i * fc;
+        if (px < 0 || px >= a.vol_x || pz < 0 || pz >= a.vol_z) continue;
+        const double fx = (int)px + 0.5 - a.vol_x * 0.5;
+        const double fz = (int)pz + 0.5 - a.vol_z * 0.5;
+        double num[RP_ROWS], den[RP_ROWS];
+#pragma unroll
+        for (int r = 0; r < RP_ROWS; r++) num[r] = den[r] = 0.0;
+        for (int k = 0; k < a.n_range; k++) {
+            const double u = fx * a.cos_t[k] + fz * a.sin_t[k] + cx;
+            if (u < 0 || u > last) continue;
+            const float* img = projs + (size_t)(a.first + k) * a.proj_y * a.proj_x + (int)u;
+#pragma unroll
+            for (int r = 0; r < RP_ROWS; r++) {
+                const float v = img[(size_t)min(y0 + r, a.proj_y - 1) * a.proj_x];
+                if (v < kEmpty) continue;
+                num[r] += v * a.cos_t[k] * a.weight[k];
+                den[r] += a.weight[k];
+            }
         }
-        if (x < a.proj_x)
-            out[(size_t)(y0 + r) * a.proj_x + x] = ((float)n < a.min_count) ? kSentinel : (float)(t / n);
+#pragma unroll
+        for (int r = 0; r < RP_ROWS; r++) {
+            if (den[r] < 0.001) continue;
+            const double v = num[r] / den[r];
+            if ((float)v <= kEmpty) continue;
+            sum[r] += v;
+            cnt[r] += 1;
+        }
     }
+    reproj_store(a, sum, cnt, sums, y0, x, out);
 }
 
 // Columns that a segment of n samples reaches at most, over the tilts: 64
@@ -231,6 +302,11 @@ void launch_reproj(const ReprojArgs& args, const float* projs, float* out, hipSt
     ReprojArgs a = args;
     const int entry = RP_ROWS * (int)sizeof(float) * a.n_range;
     auto bytes = [&](int n) { return (size_t)(std::min(reach(a, n), (double)a.proj_x) + 1.0) * entry; };
+    if (bytes(1) > (size_t)RP_LDS_MAX) {
+        hipLaunchKernelGGL(k_reproj_far, dim3((a.proj_x + 63) / 64, (a.proj_y + RP_ROWS - 1) / RP_ROWS),
+                           dim3(64 * RP_WAVES), 0, s, projs, a, out);
+        return;
+    }
     // the longest equal segments that fit; a lone reference far from a steep
     // projection spreads 64 columns over thousands and takes more LDS
     const size_t limit = bytes(1) <= (size_t)RP_LDS ? RP_LDS : RP_LDS_MAX;
@@ -238,8 +314,7 @@ void launch_reproj(const ReprojArgs& args, const float* projs, float* out, hipSt
     while (n_seg < a.ray && bytes((a.ray + n_seg - 1) / n_seg) > limit) n_seg++;
     a.seg = std::max(1, (a.ray + n_seg - 1) / n_seg);
     a.width = (int)(bytes(a.seg) / entry);
-    const size_t sums = (size_t)RP_WAVES * RP_ROWS * 64 * (sizeof(double) + sizeof(int));
-    const size_t shm = std::max((size_t)a.width * entry, sums);
+    const size_t shm = std::max((size_t)a.width * entry, (size_t)RP_SUMS);
     launch_n<REPROJ_MAX_TILTS>(a, shm, projs, out, s);
 }
 
