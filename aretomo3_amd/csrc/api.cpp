@@ -211,7 +211,7 @@ static atr_status plan_sizes(const atr_series_desc* d, Plan& p)
             !make_fft(p.vol_z, f) || !make_fft(p.vol_x, f))
             return fail(ATR_ERR_UNSUPPORTED_SIZE,
                         "WBP: ProjX, VolX or VolZ has no FFT plan");
-        if (p.vol_x > 2048 || p.vol_z > 2048)
+        if (p.vol_x > WBP_MAX || p.vol_z > WBP_MAX)
             return fail(ATR_ERR_UNSUPPORTED_SIZE,
                         "WBP supports ProjX (= VolX) <= 2048 and VolZ <= 2048");
         // slab of slices whose spectra are buffered between the WBP kernels

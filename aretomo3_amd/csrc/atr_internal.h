@@ -27,6 +27,7 @@ enum { BP_SQUARE = 0, BP_GRID = 1, BP_WIDE = 2 };
 constexpr int BP_TX = 64;
 constexpr int BP_WAVES = 4;
 constexpr int BP_THREADS = 64 * BP_WAVES;
+constexpr int WBP_MAX = 2048;                // ProjX (= VolX) and VolZ of the WBP at most
 constexpr int BP_WBP_CHUNK = 32;             // tilts staged in LDS at once, WBP grid
 constexpr int XCDS = 8;                      // workgroups go to the XCDs in turn
 // Slices from which one XCD takes all tiles of a slice (6 % of the

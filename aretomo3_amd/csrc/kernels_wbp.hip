@@ -644,11 +644,12 @@ static void launch_filter_t(const Plan& p, const float* in, hipStream_t s)
     const size_t ts = src0.tilt_stride, rs = src0.row_stride;
     if (with_pow2(p.proj, [&](auto nc) {
             constexpr int N = decltype(nc)::value;
-            hipLaunchKernelGGL((k_filter_reg<S, N>), row_grid<N>((p.vol_y + 1) / 2, p.n),
-                               dim3(fft_row_threads(N)), row_lds<N>(), s, src, ts, rs,
-                               src0.fill ? 1 : 0, p.d_fill_aln, (const double2*)p.d_tilt_stats, p.d_cs,
-                               p.n, p.vol_y, p.vol_z, p.d_tw_proj, p.d_filter, (S*)p.d_sino,
-                               p.sino_stride, p.d_sflag);
+            if constexpr (N <= WBP_MAX)
+                hipLaunchKernelGGL((k_filter_reg<S, N>), row_grid<N>((p.vol_y + 1) / 2, p.n),
+                                   dim3(fft_row_threads(N)), row_lds<N>(), s, src, ts, rs,
+                                   src0.fill ? 1 : 0, p.d_fill_aln, (const double2*)p.d_tilt_stats,
+                                   p.d_cs, p.n, p.vol_y, p.vol_z, p.d_tw_proj, p.d_filter,
+                                   (S*)p.d_sino, p.sino_stride, p.d_sflag);
         }))
         return;
     dim3 grid((p.vol_y + 1) / 2, p.n);
@@ -669,7 +670,7 @@ void launch_wbp_rowfft(const Plan& p, int ny, hipStream_t s)
 {
     if (with_pow2(2 * p.vol_x, [&](auto nc) {
             constexpr int N = decltype(nc)::value;
-            if constexpr (N <= 4096)   // VolX <= 2048
+            if constexpr (N <= 2 * WBP_MAX)
                 hipLaunchKernelGGL(k_wbp_rowfft_reg<N>, row_grid<N>(p.vol_z, ny),
                                    dim3(fft_row_threads(N)), 0, s, p.d_wbp_grid, p.vol_z, p.wbp_kb,
                                    p.d_tw_x2, p.d_wbp_t);
@@ -693,9 +694,10 @@ void launch_wbp_rowc2r(const Plan& p, int y0, int ny, float* out, hipStream_t s)
 {
     if (with_pow2(p.vol_x, [&](auto nc) {
             constexpr int N = decltype(nc)::value;
-            hipLaunchKernelGGL(k_wbp_rowc2r_reg<N>, row_grid<N>((p.vol_z + 1) / 2, ny),
-                               dim3(fft_row_threads(N)), row_lds<N>(), s, p.d_wbp_u, p.vol_y, p.vol_z,
-                               y0, p.wbp_kb, p.d_tw_x, p.layout, out);
+            if constexpr (N <= WBP_MAX)
+                hipLaunchKernelGGL(k_wbp_rowc2r_reg<N>, row_grid<N>((p.vol_z + 1) / 2, ny),
+                                   dim3(fft_row_threads(N)), row_lds<N>(), s, p.d_wbp_u, p.vol_y,
+                                   p.vol_z, y0, p.wbp_kb, p.d_tw_x, p.layout, out);
         }))
         return;
     dim3 grid((p.vol_z + 1) / 2, ny);
