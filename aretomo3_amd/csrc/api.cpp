@@ -300,7 +300,7 @@ static atr_status sart_tables_host(Plan& p, int tz, int chunk, int bz, int pf)
     parallel_for(p.n_subsets, [&](int sb) {
         const int f0 = p.subset_fp_off[sb], f1 = p.subset_fp_off[sb + 1];
         fp_pair_schedule(g, p.subset_fp.data() + f0, f1 - f0, p.proj,
-                         fp_group(p.proj, f1 - f0, waves), part[sb], waves);
+                         fp_group(p.proj, f1 - f0, waves), part[sb], p.fp_pf);
     });
     for (int sb = 0; sb < p.n_subsets; sb++) {
         p.subset_pair_off.push_back((int)sched.size());

@@ -485,7 +485,7 @@ int fp_group(int proj, int n_list, int n_waves = FP_WAVES);
 // fn(0) .. fn(n - 1) on up to 16 host threads (returns when all are done).
 void parallel_for(int n, const std::function<void(int)>& fn);
 void fp_pair_schedule(const Geometry& g, const int* list, int n_list, int proj, int group,
-                      std::vector<int>& tab, int n_waves = FP_WAVES);
+                      std::vector<int>& tab, int pf);
 void split_items(int n_items, int n_splits, std::vector<int>& starts, std::vector<int>& sizes);
 void fill_table(uint64_t seed, int n, std::vector<int>& table);
 bool ps_local_fast(const float* axis_deg, const float* local, int n, int n_patches, int in_x, int in_y,

@@ -533,16 +533,18 @@ int fp_group(int proj, int n_list, int n_waves)
 // tab gets one block of FP_WAVES * FP_MAXP entries per group of `group`
 // tilts: entry [w * FP_MAXP + i] = (local tilt << 24) | (tilt * ntile +
 // tile), the second part being the pair's row of band descriptors, or -1.
-// Only waves 0 .. n_waves - 1 get pairs (the band-prefetching projector
-// keeps its last wave for the loads).
+// pf: the projector's staging.  Only waves 0 .. fp_waves(pf) - 1 get pairs (the
+// band-prefetching projector keeps its last wave for the loads).
 void fp_pair_schedule(const Geometry& g, const int* list, int n_list, int proj, int group,
-                      std::vector<int>& tab, int n_waves)
+                      std::vector<int>& tab, int pf)
 {
+    const int n_waves = fp_waves(pf);
     const int ntile = (proj + FP_WAVE - 1) / FP_WAVE;
     const int nb = g.fp_nbands;
     // two workgroups per CU: one fills the other's waits, exchanges give less than
-    // 1 % there (and take a third of the plan's time)
-    const bool two = fp_lds_bytes(g.fp_bz, proj, 0) <= (size_t)FP_LDS_TWO;
+    // 1 % there (and take a third of the plan's time).  The prefetching
+    // projectors have one, whatever their bands.
+    const bool two = pf == 0 && fp_lds_bytes(g.fp_bz, proj, 0) <= (size_t)FP_LDS_TWO;
     for (int j0 = 0; j0 < n_list; j0 += group) {
         const int ng = std::min(group, n_list - j0);
         const int n_items = ng * ntile;
