@@ -389,11 +389,12 @@ struct FpItem {
 
 // Batched forward projection: one persistent launch per staging variant
 // present in a set of queue entries (each variant's kernel holds only its
-// own code, as the per-series kernels do), then one launch of the
-// empty-voxel variant over every entry, whose blocks leave at once on slices
-// without empty voxels.  Variants 0-3: band prefetch by DMA, 4-7: direct
-// staging (VolX 512, 1024, 2048, any), 8-9: register prefetch (VolX 1024,
-// 2048).
+// own code, as the per-series kernels do), and one launch of the empty-voxel
+// variant over every entry, whose blocks leave at once on slices without
+// empty voxels.  Variants 0-3: band prefetch by DMA (VolX 512, 1024, 2048,
+// any); 4, 5, 7: direct staging, two workgroups per CU (VolX 512, 1024, any);
+// 6 and FP_VARIANT_ANY: direct staging, one per CU (VolX 2048, any); 8-9:
+// register prefetch (VolX 1024, 2048).
 constexpr int FP_VARIANT_EMPTY = 10;
 constexpr int FP_VARIANT_ANY = 11;
 constexpr int FP_VARIANTS = 12;

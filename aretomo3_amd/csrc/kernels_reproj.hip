@@ -28,9 +28,13 @@ namespace atr {
 // segment whose staged columns hold an empty value takes the general path,
 // which counts each row's samples by itself.
 //
-// 1024^2 x 256, 8 reference tilts at 48 degrees: 0.81 ms, bound by FP64 issue
-// (5.3 ms with the slice formed in memory and read back, where every voxel of
-// it cost its coordinates and a division).
+// 1024^2 x 256, 8 reference tilts at 48 degrees: 0.68 ms (0.81 with the rays'
+// sums written in the kernel's own body: 84 more reads of spilled scalars; 5.3
+// with the slice formed in memory and read back, where every voxel of it cost
+// its coordinates and a division).  Bound by VALU issue, busy 0.82 of the time:
+// 59 instructions per sample and tilt, 16 of them FP64 arithmetic (8 for the
+// rows, the others for coordinates), 8 conversions, the rest compares, picks,
+// addresses and spilled scalars.
 constexpr int RP_ROWS = 8;
 constexpr int RP_WAVES = 4;
 constexpr int RP_LDS = 52 * 1024;      // three workgroups per CU
