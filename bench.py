@@ -676,7 +676,7 @@ def extras_bench(args):
     synchronize()
     ms_r = 1e3 * (time.perf_counter() - t0) / len(jobs)
     nr = np.mean([b - a + 1 for _, _, (a, b) in jobs])
-    bytes_r = 4.0 * nr * px * px + 2 * 4.0 * (2 * px) * vz * px + 4.0 * px * px
+    bytes_r = 4.0 * nr * px * px + 4.0 * px * px   # references in, projection out
     rows = 8
     sub = np.ascontiguousarray(projs[:, px // 2 - rows // 2: px // 2 + rows // 2])
     idx, skip, _ = jobs[len(jobs) // 2]
