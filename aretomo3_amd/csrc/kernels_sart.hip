@@ -704,7 +704,9 @@ __global__ __launch_bounds__(BP_THREADS, 6) void k_wbp_grid_bp(const BpArgs* __r
 // (series, slice, run of BP_ITEM_TILES tiles) items from a queue; entries
 // are ordered by their first item.  One launch runs one tile shape (0: 16 z rows x 16 tilts
 // per stage, 1: 16 x 8, 2: 8 x 16, 3: 8 x 8), so each shape's kernel holds
-// only its own code and registers, as the per-series kernels do.
+// only its own code and registers.  Shape 0 takes 97 VGPRs, 4 waves per SIMD
+// (k_back_proj<float, 16, 16>: 87, and 5): 16 uneven series spend 300 ms here,
+// 250 series by series.
 template <typename S, int SHAPE>
 __global__ __launch_bounds__(BP_THREADS) void k_back_proj_batch(const BpItem* __restrict__ e, int n_e,
                                                            int total, int* __restrict__ counter)
